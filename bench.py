@@ -607,7 +607,7 @@ def main():
         time.perf_counter() - t, info.nfluid, info.nwall, info.ncorner, info.device_bytes / 1e9))
     nc = info.nc8 * 8
     flow = info.sweep_path == 2
-    log("sweep: %s" % ("one launch per iteration (k_sweep_flow)" if flow else "one launch per hyperplane"))
+    log("sweep: %s" % ("one launch per iteration (k_sweep_pencil)" if flow else "one launch per hyperplane"))
     if args.warmup:
         s.iterate(args.warmup)
     log("warm-up done (%d steps)" % args.warmup)
@@ -642,8 +642,8 @@ def main():
     wl = "spheres200_phi040_kn1_v8"
     roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "traffic": traffic_from_profiles(wl + ("_flow" if flow else "")),
-            "kernel": "k_sweep_flow" if flow else "k_sweep1<double, false>",
+            "traffic": traffic_from_profiles(wl + ("_rows" if flow else "")),
+            "kernel": "k_sweep_pencil" if flow else "k_sweep1<double, false>",
             "bytes_per_update": bytes_per_update,
             "sweep_ms_per_step": round(ms[0] / args.steps, 4)}
     cpu = None

@@ -1,12 +1,10 @@
 """Autotuner of the sweep schedule per request class.
 
-One source iteration's sweep is a chain of dependent launches: one per
-oriented hyperplane (i + j + k = const, all octants), or, with the tiled
-schedule, one per tile diagonal, each wave walking a tile of tx * ty * tz
-cells of one octant plane by plane.  Which is faster depends on the request:
-large images keep every launch full and favour the hyperplane sweep's short
-waves; small ones are bound by the launch chain's length, which tiles cut by
-their side.  This module times every candidate schedule on a representative
+One source iteration's sweep is one launch that takes the image row by row
+(the library's default), or a chain of dependent launches: one per oriented
+hyperplane (i + j + k = const, all octants), or, with the tiled schedule, one
+per tile diagonal, each wave walking a tile of tx * ty * tz cells of one
+octant plane by plane.  This module times every candidate schedule on a representative
 request of each class of the serving stream (cube side, velocity grid:
 seeded sphere pack at porosity 0.4, Kn 1, 4 fluid layers, wallExtOrder 2)
 and keeps the fastest per class in a table (JSON).  Server.submit applies the
@@ -41,19 +39,21 @@ def tile_shape(code):
     return code & 255, (code >> 8) & 255, code >> 16
 
 
-# (sweep, tile) candidates: the hyperplane sweep and tiled sweeps (the tiled
+# (sweep, tile) candidates: the default, the hyperplane sweep and tiled sweeps (the tiled
 # kernel serves grids of at most 64 velocities per octant)
 TILES = [tile_code(*t) for t in ((2, 2, 2), (2, 2, 4), (4, 2, 4), (4, 4, 4), (4, 2, 8), (4, 4, 8))]
 
 
 def candidates(nc):
-    c = [(1, 0)]
+    c = [(0, 0), (1, 0)]
     if nc ** 3 <= 64:
         c += [(2, t) for t in TILES]
     return c
 
 
 def label(sweep, tile):
+    if sweep == 0:
+        return "rows"
     if sweep == 1:
         return "hyperplanes"
     return "tiles %dx%dx%d" % tile_shape(tile)

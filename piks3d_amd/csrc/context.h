@@ -22,9 +22,11 @@ struct Dims {
   int Nx, Ny, Nz, Nxt;
   int64_t Nxyt, Ntotal;
   int Nc8;
+  int vs;                  // elements per slot of f: Nc8, padded for the pencil sweep
   // storage of f: octant o keeps its cells in family ofam(o)'s order, pos[F]
-  // maps a cell to that order (unstored cells to the zero slot); ostride =
-  // elements per octant
+  // maps a cell to that order (unstored cells to the zero slot; the same map
+  // four times for the pencil sweep's raster order); ostride = elements per
+  // octant
   const int32_t* pos[4];
   int64_t ostride;
   // right-hand sides (Knudsen numbers) sharing the geometry: kernels take the
@@ -113,23 +115,17 @@ struct Ctx {
   bool sweep_recip = false;    // fast mode: multiply by a tabulated 1 / denominator
   bool sweep_generic = false;  // single solve through the multi-right-hand-side kernel
   int sweep_nt = 1;            // tasks per wave of the single-solve sweep (k_sweep1)
-  // single-launch sweep (k_sweep_flow; FP64 iterations of a single solve with
-  // 64 velocities per octant on a context with its own stream): octant o on
-  // XCD o, tasks split statically over flow_waves waves per octant, or claimed
-  // from a counter when the octant's waves are not all resident
+  // pencil sweep (k_sweep_pencil): the whole sweep in one launch, octant o on
+  // XCD o, rows of cells along x claimed in dependency order
   int flow_req = -1;                  // -1 where it applies, 0 off, 1 required
-  bool sweep_flow = false;            // in use
-  int flow_waves = 0;
-  int flow_barrier = 1 << 12;         // polls for an octant's waves to arrive
-  int flow_early_req = -1;            // early upwind loads: -1 by size, 0 off, 1 on
-  int flow_strips = 1;                // bands of y an octant sweeps one after another
-  bool flow_early = false;
-  TaskRec* flow_rec = nullptr;        // octant-major tasks (flow_setup)
-  int64_t flow_off[9] = {};
-  uint32_t* flow_flags = nullptr;     // [octant][slot]
-  uint32_t* flow_epoch = nullptr;     // the launch's state (k_flow_epoch)
-  uint32_t* flow_err = nullptr;
-  uint32_t* flow_diag = nullptr;      // per block: octant and tasks done (the failure message)
+  int flow_strips = 0;                // strips of y rows asked for (0: by size)
+  bool pencil = false;                // in use
+  int pen_rows = 0;                   // y rows per strip
+  int pen_waves = 0;                  // waves launched per octant
+  TaskRec* pen_rec = nullptr;         // Geometry::pen_rec
+  Geometry::Pencil* pen_list = nullptr;  // Geometry::pen
+  uint32_t* pen_prog = nullptr;       // [unit][octant][row]: progress
+  uint32_t* pen_state = nullptr;      // the launch's state (k_pencil_begin)
   int multi_rb = 0;            // right-hand sides per wave of the several-Kn sweep (0: 1,
                                // measured fastest: 1, 2, 4 took 14.1, 14.8, 16.1 s on 16 Kn)
   int oct_groups = 0;          // octant groups of the sweep (1, 2, 4, 8; 0: 4 on a context
@@ -207,6 +203,12 @@ int ctx_enqueue(Ctx& c, int nsteps);
 // Enqueue the copy of Ux on the plane x = 2 (Ny*Nz doubles per right-hand
 // side, j fastest) into host memory (pinned, so the copy is asynchronous).
 int ctx_enqueue_plane(Ctx& c, double* host_plane);
+// Enqueue the copy of the sweep's failure state (kPenErrWords words, after
+// the iterations enqueued so far) into host memory (pinned), and read it once
+// the copy is done: 0, or a PIKS_E_* code with the message set.
+constexpr int kPenErrWords = 6;
+int ctx_enqueue_state(Ctx& c, uint32_t* host_words);
+int ctx_state_check(const Ctx& c, const uint32_t* host_words);
 // Mass flow through x = 2 from one right-hand side's plane, in the
 // reference's summation order (massLocal of src/output.F90:80-142).
 double ctx_mass(const Ctx& c, const double* plane);

@@ -387,22 +387,175 @@ int build_geometry(const GeomInput& in, const uint8_t* raw, int64_t nbytes, Geom
     err = "domain of " + std::to_string(g.Ntotal) + " cells (with ghosts) is too large";
     return PIKS_E_ARG;
   }
+  if (in.pencil_rows > 0 && build_pencil_schedule(g, in.pencil_rows, in.pencil_vs, threads)) return PIKS_OK;
   build_sweep_schedule(g, threads);
   return PIKS_OK;
 }
 
+const std::vector<int32_t>& Geometry::opos(int o) const { return pos[raster ? 0 : ofam(o)]; }
+
 void build_wall_positions(Geometry& g, int threads);
 
+namespace {
+
+// Whether a cell is stored (see Geometry::nstore), for i in [0, Nx + 1].
+bool is_stored(const Geometry& g, int i, int j, int k) {
+  const uint8_t l = g.lab[(size_t)g.cell(i, j, k)];
+  const bool plane = i <= 1 || i >= g.Nx || j == 1 || j == g.Ny || k == 1 || k == g.Nz;
+  return plane || l == FLUID || l >= 20;
+}
+
+}  // namespace
+
+bool build_pencil_schedule(Geometry& g, int rows, int vs, int threads) {
+  const int Nx = g.Nx, Ny = g.Ny, Nz = g.Nz;
+  const int64_t npen = (int64_t)Ny * Nz;
+  g.raster = true;
+  // raster storage order: the stored cells of every row, rows joined in order
+  std::vector<int64_t> row0((size_t)npen + 1, 0);
+  parallel_for(Nz, threads, [&](int kk) {
+    for (int j = 1; j <= Ny; ++j) {
+      int64_t n = 0;
+      for (int i = 0; i <= Nx + 1; ++i) n += is_stored(g, i, j, kk + 1);
+      row0[(size_t)((j - 1) + (int64_t)kk * Ny) + 1] = n;
+    }
+  });
+  for (int64_t q = 0; q < npen; ++q) row0[(size_t)q + 1] += row0[(size_t)q];
+  const int64_t ns = g.nstore = row0[(size_t)npen];
+  if (8 * (ns + 1) >= (int64_t)Geometry::kPenFw || (int64_t)g.ncorner * 8 >= (int64_t)Geometry::kPenFw ||
+      Nx + 1 >= 1 << 14)
+    return false;
+  std::vector<int32_t>& pos = g.pos[0];
+  pos.assign((size_t)g.Ntotal, (int32_t)ns);
+  parallel_for(Nz, threads, [&](int kk) {
+    for (int j = 1; j <= Ny; ++j) {
+      int64_t at = row0[(size_t)((j - 1) + (int64_t)kk * Ny)];
+      for (int i = 0; i <= Nx + 1; ++i)
+        if (is_stored(g, i, j, kk + 1)) pos[(size_t)g.cell(i, j, kk + 1)] = (int32_t)at++;
+    }
+  });
+  // rows of each octant in the order they are taken, their tasks counted
+  std::vector<Geometry::Pencil> per[8];
+  std::atomic<int> bad{0};
+  parallel_for(8, threads, [&](int o) {
+    std::vector<Geometry::Pencil>& v = per[o];
+    for (int j0 = 0; j0 < Ny; j0 += rows) {
+      const int j1 = std::min(Ny, j0 + rows);
+      for (int s = j0; s <= j1 - 1 + Nz - 1; ++s)
+        for (int oj = std::max(j0, s - (Nz - 1)); oj < j1 && oj <= s; ++oj) {
+          const int ok = s - oj;
+          if (oj < 1 || ok < 1) continue;  // the octant's inflow layers are not swept
+          const int j = osy(o) > 0 ? oj + 1 : Ny - oj, k = osz(o) > 0 ? ok + 1 : Nz - ok;
+          const int64_t c = g.cell(1, j, k);
+          uint32_t n = 0;
+          for (int i = osx(o) > 0 ? 2 : 1, e = osx(o) > 0 ? Nx : Nx - 1; i <= e; ++i)
+            n += g.lab[(size_t)(c + i - 1)] == FLUID;
+          if (!n) continue;
+          // the rows it reads: its own, two upwind in y, two in z
+          const int64_t id = (j - 1) + (int64_t)(k - 1) * Ny;
+          int64_t lo = id, hi = id;
+          for (int d = 1; d <= 2; ++d) {
+            if (oj >= d) lo = std::min(lo, id - d * osy(o)), hi = std::max(hi, id - d * osy(o));
+            if (ok >= d) lo = std::min(lo, id - (int64_t)d * osz(o) * Ny), hi = std::max(hi, id - (int64_t)d * osz(o) * Ny);
+          }
+          const int64_t len = row0[(size_t)hi + 1] - row0[(size_t)lo];
+          if (len * vs >= (int64_t)1 << 28) bad = 1;
+          v.push_back(Geometry::Pencil{0, n, (uint32_t)id, (uint32_t)(c - 1), (uint32_t)row0[(size_t)lo], (uint32_t)len, {}});
+        }
+    }
+  });
+  g.pen.clear();
+  int64_t at = 0;
+  for (int o = 0; o < 8; ++o) {
+    g.pen_off[o] = (int64_t)g.pen.size();
+    const int64_t first = at;
+    for (Geometry::Pencil p : per[o]) {
+      p.rec = (uint32_t)at;
+      at += p.n;
+      g.pen.push_back(p);
+    }
+    g.pen_tasks[o] = at - first;
+  }
+  g.pen_off[8] = (int64_t)g.pen.size();
+  if (bad || at >= ((int64_t)1 << 30)) return false;
+  g.pen_rec.resize((size_t)at * Geometry::kTaskWords);
+  const int kChunk = 256;
+  for (int o = 0; o < 8; ++o) {
+    const int64_t p0 = g.pen_off[o], np = g.pen_off[o + 1] - p0;
+    const int dx = osx(o);
+    const int64_t st[2] = {(int64_t)osy(o) * g.Nxt, (int64_t)osz(o) * g.Nxyt};
+    const uint32_t wait[2] = {Geometry::kPenWaitY, Geometry::kPenWaitZ};
+    parallel_for((int)((np + kChunk - 1) / kChunk), threads, [&](int chunk) {
+      for (int64_t q = p0 + (int64_t)chunk * kChunk; q < p0 + std::min(np, (int64_t)(chunk + 1) * kChunk); ++q) {
+        Geometry::Pencil& p = g.pen[(size_t)q];
+        const int j = 1 + (int)(p.id % (uint32_t)Ny), k = 1 + (int)(p.id / (uint32_t)Ny);
+        const int on[2] = {osy(o) > 0 ? j - 1 : Ny - j, osz(o) > 0 ? k - 1 : Nz - k};
+        // element offset of a storage index in the row's window
+        auto rel = [&](int32_t at) -> uint32_t {
+          return (uint32_t)((at == (int32_t)ns ? (int64_t)p.len : (int64_t)at - p.lo) * vs);
+        };
+        uint32_t* r = &g.pen_rec[(size_t)p.rec * Geometry::kTaskWords];
+        uint32_t waits = 0;
+        for (int oi = 1; oi < Nx; ++oi) {
+          const int i = dx > 0 ? oi + 1 : Nx - oi;
+          const int64_t c = (int64_t)p.cell + i;
+          if (g.lab[(size_t)c] != FLUID) continue;
+          const uint32_t cc = g.code[(size_t)c];
+          uint32_t w0 = rel(pos[(size_t)c]) | ((cc >> (3 * o)) & 7u) << 28;
+          uint32_t w1 = (uint32_t)i | (uint32_t)(oi + 1) << 14;
+          const bool x1 = oi - 1 >= 1 && g.lab[(size_t)(c - dx)] == FLUID;
+          const bool x2 = oi - 2 >= 1 && g.lab[(size_t)(c - 2 * dx)] == FLUID;
+          r[6] = x1 ? 0u : rel(pos[(size_t)(c - dx)]) * 8u;
+          r[7] = x1 || x2 ? 0u : rel(pos[(size_t)(c - 2 * dx)]) * 8u;
+          w1 |= (x1 ? Geometry::kPenX1Reg : 0u) | (x2 ? Geometry::kPenX2Reg : 0u);
+          for (int ax = 0; ax < 2; ++ax) {
+            bool swept1 = false;
+            for (int d = 1; d <= 2; ++d) {
+              const int64_t n = c - d * st[ax];
+              uint32_t w = rel(pos[(size_t)n]) * 8u;
+              if (on[ax] - d >= 1 && g.lab[(size_t)n] == FLUID) {
+                if (d == 1) {
+                  w1 |= wait[ax];
+                  swept1 = true;
+                } else if (!swept1) {
+                  r[7] |= ax == 0 ? Geometry::kPenWaitY2 : Geometry::kPenWaitZ2;
+                  w0 |= Geometry::kPenSpecial;
+                }
+              } else if ((cc >> (24 + o)) & 1u) {  // reads a wall slot the reference switched
+                const int64_t f = flow_switched_word(g, o, n, ax + 1);
+                if (f == -2) bad = 1;
+                if (f >= 0) {
+                  const uint32_t x = (uint32_t)(f >> 28) & 7u, idx = (uint32_t)f & 0x0fffffffu;
+                  w = (f >> 31) & 1 ? idx | Geometry::kPenFar | Geometry::kPenFw
+                                    : (uint32_t)((int64_t)((uint32_t)o ^ x) * (ns + 1) + idx) | Geometry::kPenFar;
+                  w0 |= Geometry::kPenSpecial;
+                }
+              }
+              r[2 + 2 * ax + d - 1] = w;
+            }
+          }
+          waits |= w1;
+          r[0] = w0;
+          r[1] = w1;
+          r += Geometry::kTaskWords;
+        }
+        p.n |= (waits & Geometry::kPenWaitY ? 1u << 31 : 0u) | (waits & Geometry::kPenWaitZ ? 1u << 30 : 0u);
+      }
+    });
+  }
+  if (bad) return false;
+  build_wall_positions(g, threads);
+  return true;
+}
+
 void build_sweep_schedule(Geometry& g, int threads) {
+  g.raster = false;
   // cells that are stored
   std::vector<uint8_t> stored((size_t)g.Ntotal, 0);
   for (int k = 1; k <= g.Nz; ++k)
     for (int j = 1; j <= g.Ny; ++j)
-      for (int i = 0; i <= g.Nx + 1; ++i) {
-        const uint8_t l = g.lab[(size_t)g.cell(i, j, k)];
-        const bool plane = i <= 1 || i >= g.Nx || j == 1 || j == g.Ny || k == 1 || k == g.Nz;
-        if (plane || l == FLUID || l >= 20) stored[(size_t)g.cell(i, j, k)] = 1;
-      }
+      for (int i = 0; i <= g.Nx + 1; ++i)
+        if (is_stored(g, i, j, k)) stored[(size_t)g.cell(i, j, k)] = 1;
   int64_t ns = 0;
   for (uint8_t v : stored) ns += v;
   g.nstore = ns;
@@ -669,7 +822,7 @@ bool build_tile_schedule(Geometry& g, int TX, int TY, int TZ, int threads) {
 std::vector<uint32_t> build_nonswept(const Geometry& g, int threads) {
   std::vector<std::vector<uint32_t>> per(8);
   parallel_for(8, threads, [&](int o) {
-    const std::vector<int32_t>& pos = g.pos[ofam(o)];
+    const std::vector<int32_t>& pos = g.opos(o);
     std::vector<uint32_t>& out = per[(size_t)o];
     for (int k = -1; k <= g.Nz + 2; ++k)
       for (int j = -1; j <= g.Ny + 2; ++j)
@@ -702,13 +855,13 @@ void build_wall_positions(Geometry& g, int threads) {
     for (size_t w = (size_t)chunk * 4096; w < std::min(nwall, (size_t)(chunk + 1) * 4096); ++w) {
       const int64_t c = g.wall_cell[w];
       int32_t* q = &g.wall_pos[w * K];
-      for (int F = 0; F < 4; ++F) q[F] = g.pos[F][(size_t)c];
+      for (int F = 0; F < 4; ++F) q[F] = g.pos[g.raster ? 0 : F][(size_t)c];
       const WallProg P = wall_prog(g.wall_label[w]);
       for (int fa = 0; fa < P.nface; ++fa)
         for (int d = 1; d <= 2; ++d)
           for (int k = 0; k < 4; ++k) {
             const int64_t n = c + (int64_t)d * P.face[fa].dir * stride[(int)P.face[fa].axis];
-            q[4 + fa * 8 + (d - 1) * 4 + k] = g.pos[ofam(P.face[fa].in[k])][(size_t)n];
+            q[4 + fa * 8 + (d - 1) * 4 + k] = g.opos(P.face[fa].in[k])[(size_t)n];
           }
     }
   });
@@ -719,7 +872,7 @@ int64_t flow_switched_word(const Geometry& g, int o, int64_t n, int axis) {
   const int w = g.wid[(size_t)n];
   const int src = (int)((g.wall_views[(size_t)w] >> (8 * o + (axis == 2 ? 4 : 0))) & 15u);
   if (src == 0) return -1;
-  if (src <= 8) return (int64_t)(uint32_t)g.pos[ofam(src - 1)][(size_t)n] | (int64_t)((src - 1) ^ o) << 28;
+  if (src <= 8) return (int64_t)(uint32_t)g.opos(src - 1)[(size_t)n] | (int64_t)((src - 1) ^ o) << 28;
   const int64_t corner = g.wall_corner[(size_t)w];
   if (corner < 0 || corner * 8 + o >= (1 << 28)) return -2;
   return (corner * 8 + o) | 0x90000000ll;

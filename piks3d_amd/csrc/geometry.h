@@ -25,6 +25,9 @@ struct GeomInput {
   int fluid_layer;
   int wall_ext_order;
   int threads = 0;          // host threads for the preprocessing (0: host_threads())
+  int pencil_rows = 0;      // > 0: raster storage and the pencil schedule with strips of
+                            // this many y rows, instead of the hyperplane schedule
+  int pencil_vs = 0;        // elements per slot of f (the schedule's offsets are in elements)
 };
 
 // Host threads the preprocessing of one image uses: the calling thread's
@@ -86,8 +89,12 @@ struct Geometry {
   // in the order of its family ofam(o): ascending sx*i + sy*j + sz*k with the
   // family's signs, then k, then j, so that one hyperplane of a sweep is one
   // contiguous range.  pos[F] maps a cell to its index in family F's order.
+  // With the pencil schedule (raster) every octant keeps its cells in one
+  // raster order instead (k, then j, then i), held in pos[0].
   int64_t nstore = 0;
+  bool raster = false;
   std::vector<int32_t> pos[4];
+  const std::vector<int32_t>& opos(int o) const;
 
   // Sweep schedule.  Octant o updates its swept cells (fluid cells past the
   // octant's inflow layer) in order of the oriented hyperplane
@@ -132,6 +139,48 @@ struct Geometry {
   int64_t tl_maxwin = 0;               // largest storage window (cells)
   int64_t tl_maxspan = 0;              // largest span of a tile's swept cell indices
 
+  // Pencil schedule (build_pencil_schedule; raster storage).  A pencil is a
+  // row of the grid along x: octant o updates its swept cells of the row
+  // (j, k) in its x direction, one after another, so the x upwind values are
+  // the row's own last results and a row waits on the rows (j -+ 1, k) and
+  // (j, k -+ 1) only.  pen holds the rows with swept cells, octant-major
+  // (pen_off[o]), each after the rows it reads: strip by strip of y (strip
+  // rows each, in the octant's y direction), within a strip by oj + ok, then
+  // oj.  pen_rec holds their tasks, kTaskWords words each, row by row.  Offsets
+  // are elements of f from the row's window (the stored cells from the first
+  // to the last row a task reads), the zero slot the window's end:
+  //   [0] the slot's offset | first-order flags << 28 (bits 0-2: x, y, z) |
+  //       kPenSpecial (a far source, or a wait at distance 2)
+  //   [1] x index i | (oriented x + 1) << 14 | kPenX1Reg, kPenX2Reg (the x
+  //       upwind value at distance 1, 2 is the row's own result) | kPenWaitY,
+  //       kPenWaitZ (the neighbour at distance 1 is swept: wait for its row)
+  //   [2..5] the y upwind sources at distance 1 and 2, then z: offsets in
+  //       bytes of 8-byte elements, or kPenFar (beyond every window): a storage
+  //       row octant * (nstore + 1) + index, or with kPenFw a corner store
+  //       entry corner * 8 + octant (where the reference switched a wall slot)
+  //   [6], [7] the x sources at distance 1 and 2 where they are no register,
+  //       offsets in bytes of 8-byte elements; in the low bits of [7]
+  //       kPenWaitY2, kPenWaitZ2 (the neighbour at distance 2 is swept and the
+  //       one at distance 1 is not: wait for its row)
+  // x upwind values are kept as the last two: a task after a swept one shifts
+  // them, a task that starts a run loads them (the value at distance 2 being
+  // the last result where kPenX2Reg says so).
+  struct alignas(32) Pencil {
+    uint32_t rec;             // first task
+    uint32_t n;               // tasks | some task waits on y << 31, on z << 30
+    uint32_t id;              // (j - 1) + (k - 1) * Ny
+    uint32_t cell;            // the row's cell at x = 0
+    uint32_t lo, len;         // window: first storage index, cells
+    uint32_t pad[2];
+  };
+  static constexpr uint32_t kPenSpecial = 1u << 31;
+  static constexpr uint32_t kPenX1Reg = 1u << 28, kPenX2Reg = 1u << 29, kPenWaitY = 1u << 30, kPenWaitZ = 1u << 31;
+  static constexpr uint32_t kPenFar = 1u << 31, kPenFw = 1u << 30, kPenWaitY2 = 1, kPenWaitZ2 = 2;
+  std::vector<Pencil> pen;
+  std::vector<uint32_t> pen_rec;
+  int64_t pen_off[9] = {};
+  int64_t pen_tasks[8] = {};
+
   int64_t cell(int i, int j, int k) const {
     return (int64_t)(i + 1) + (int64_t)(j + 1) * Nxt + (int64_t)(k + 1) * Nxyt;
   }
@@ -143,6 +192,11 @@ int build_geometry(const GeomInput& in, const uint8_t* raw, int64_t nbytes, Geom
 
 // Fill the storage order (nstore, pos) and the sweep schedule (hp_task, hp_off).
 void build_sweep_schedule(Geometry& g, int threads);
+
+// Fill the raster storage order and the pencil schedule (pen, pen_rec), with
+// strips of `rows` y rows and vs elements per slot.  False if the image is beyond the records' limits
+// (the hyperplane schedule is then built over it).
+bool build_pencil_schedule(Geometry& g, int rows, int vs, int threads);
 
 // Dword positions inside the tiled sweep's records (tile of tx * ty cells per
 // plane, ns = tx * ty slots, slot s = b * tx + a for oriented offsets a, b).

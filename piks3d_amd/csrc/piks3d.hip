@@ -2,10 +2,12 @@
 // voxel image, behind the C ABI in include/piks3d.h.
 //
 // One source iteration of the reference (src/solver.F90:111-1940) becomes:
-//   sweep      8 octants at once; one launch per oriented hyperplane
-//              i+j+k; a 64-lane wave updates all velocities of one (cell,
-//              octant) (f loads coalesced along the velocity index); partial
-//              moments of each (cell, octant) reduced in registers
+//   sweep      8 octants at once, one launch: octant o on XCD o, a 64-lane wave
+//              walks a row of cells along x, 64 velocities in its lanes (f
+//              loads coalesced along the velocity index), rows in dependency
+//              order; partial moments of each (cell, octant) reduced in
+//              registers.  Where that does not apply, one launch per oriented
+//              hyperplane i+j+k or per diagonal of tiles
 //   commit     the reference's in-sweep wall switches, applied after the sweep
 //              (readers were redirected to the switched sources during it)
 //   halo       periodic x exchange with the reference's one-iteration lag
@@ -13,8 +15,8 @@
 //              velocities, re-emit (diffuse + specular)
 //   in/out     pressure-drop inlet/outlet, then the four symmetry planes
 //   moments    sum of the sweep partials; recomputed from f on boundary planes
-// Device layout: f[octant][cell][velocity] over the full ghosted grid, cell =
-// (i+1) + (j+1)Nxt + (k+1)Nxt*Nyt, velocity fastest.
+// Device layout: f[octant][slot][velocity], velocity fastest, one slot per
+// stored cell (Geometry::pos) and a zero slot per octant.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -44,7 +46,7 @@ int set_error(int code, const std::string& msg) {
   return code;
 }
 
-int flow_check(Ctx& c);  // the single-launch sweep's failure flag (defined below)
+int pencil_check(Ctx& c);  // the pencil sweep's failure flag (defined below)
 
 }  // namespace piks
 
@@ -144,9 +146,28 @@ __device__ __forceinline__ T ld_const(const T* p) {
 #endif
 }
 
+// A wave-uniform pointer to data that nothing in the kernel writes, as a
+// constant-address-space pointer whose origin the compiler does not see (it
+// would fall back to vector loads through the original global pointer).
+#if defined(__HIP_DEVICE_COMPILE__)
+template <typename T>
+using ConstPtr = const __attribute__((address_space(4))) T*;
+template <typename T>
+__device__ __forceinline__ ConstPtr<T> const_ptr(const T* p) {
+  uint64_t v = (uint64_t)p;
+  asm("" : "+s"(v));
+  return (ConstPtr<T>)v;
+}
+#else
+template <typename T>
+using ConstPtr = const T*;
+template <typename T>
+__device__ __forceinline__ ConstPtr<T> const_ptr(const T* p) { return p; }
+#endif
+
 // element offset of (octant o, cell, velocity 0) in f
 __device__ __forceinline__ size_t fat(const Dims& d, int o, int64_t cell) {
-  return (size_t)o * d.ostride + (size_t)d.pos[ofam(o)][cell] * d.Nc8;
+  return (size_t)o * d.ostride + (size_t)d.pos[ofam(o)][cell] * d.vs;
 }
 
 // ------------------------------------------------------------------ sweep
@@ -158,7 +179,7 @@ template <typename T>
 struct SweepArgs {
   T* f;
   const Mom* mom;
-  double* part;            // [cell][octant][4] partial moments; null = skip
+  double* part;            // [octant][cell][4] partial moments; null = skip
   const TaskRec* tasks;    // this hyperplane's task records
   const SweepWin* win;     // this hyperplane's storage window per octant
   const double* cx;
@@ -427,7 +448,7 @@ __global__ __launch_bounds__(kThreads) void k_sweep(SweepArgs<T> a) {
         if ((lane & 15) == 0) {
           const int q = lane >> 4;
           const double sgn = q == 1 ? sx : q == 2 ? sy : q == 3 ? sz : 1;
-          double* pp = a.part + (size_t)(r0 + k) * a.rs_mom * 32 + ((size_t)cell * 8 + o) * 4 + q;
+          double* pp = a.part + (size_t)(r0 + k) * a.rs_mom * 32 + ((size_t)o * a.rs_mom + cell) * 4 + q;
           // velocity passes after the first add to the first pass's sum
           *pp = base == 0 ? sgn * z : *pp + sgn * z;
         }
@@ -566,7 +587,7 @@ __device__ __forceinline__ void sweep1_task(const SweepArgs<T>& a) {
           // octant's: bit q of neg is set when partial q is negated
           const uint32_t q = (uint32_t)lane >> 4;
           const double zz = ((kOctNeg >> (4 * o[j] + q)) & 1u) ? -z : z;
-          double* pp = partr + ((size_t)cell[j] * 8 + o[j]) * 4 + q;
+          double* pp = partr + ((size_t)o[j] * a.rs_mom + cell[j]) * 4 + q;
           // passes after the first add to the first pass's sum
           *pp = base == 0 ? zz : *pp + zz;
         }
@@ -587,436 +608,514 @@ __global__ __launch_bounds__(64) void k_sweep1_passes(SweepArgs<T> a) { sweep1_t
 template <typename T, int kDC = 0>
 __global__ __launch_bounds__(64) void k_sweep1_rhs(SweepArgs<T> a) { sweep1_task<T, false, true, kDC, 1, true>(a); }
 
-// ------------------------------------------------------------------ single-launch sweep
+// ------------------------------------------------------------------ pencil sweep
 
-// The whole sweep of one source iteration in one launch: no launch gaps
-// between hyperplanes (the default for FP64 single solves with 64
-// velocities per octant; PIKS_SWEEP_FLOW).  A block sweeps the octant
-// numbered like the XCD it runs on (its hardware XCD id), so every producer
-// and consumer of an octant's slots share one L2, and takes its arrival
-// number w in that octant from a per-XCD counter.  Tasks are in hyperplane
-// order (rec, built by the host), so a task's upwind neighbours come earlier.
-// When all W waves of an octant have arrived (the set-up probe sizes W to
-// what is resident at once), wave w takes tasks w, w + W, w + 2W, ...: the
-// earliest unfinished task can always proceed and no wait is circular.  If
-// a wave waits `barrier` polls without that happening (kernels of other
-// streams holding CUs), the octant switches to claims: every wave, late
-// ones included, takes the next task from a per-octant counter, which needs
-// no residency (a task waits only on tasks claimed before it by running
-// waves) but serialises the claims (8-12x slower when every task is
-// claimed).  A finished task sets its slot's flag to the sweep's epoch after
-// its stores have reached L2; a task waits for the flags of the nearest
-// swept upwind neighbour along each axis (their own waits cover the one
-// behind).  Flags are polled with agent-scope loads, which miss the CU's L1
-// (an L1 line polled before the flag changed would be served again: a
-// workgroup-scope invalidate leaves it).  Values are plain loads served by
-// the XCD's L2: within the launch no CU loads a slot's lines before they
-// are final (its readers wait for its flag or for the flag of a task that
-// waited for it, and its own task's read of the previous value is followed
-// by its store, which updates that CU's L1), and the L1 starts the launch
-// invalidated.  Every wait gives up after `spin` polls (a safety net: it
-// sets err and the wave ends, so the grid always drains); k_flow_done then
-// checks that every octant's tasks were done.  The update is sweep1_task's,
-// operation for operation; reads of switched wall slots come resolved in
-// the records (flow_switched_word).
-struct FlowArgs {
-  double* f;
-  const Mom* mom;
-  double* part;             // [cell][octant][4] partial moments; null = skip
-  const TaskRec* rec;       // octant-major tasks (flow_setup): word 0 the slot,
-                            // words 1..6 the upwind sources (flow_source)
-  uint32_t* flags;          // [octant][slot]: epoch of the last update
-  const uint32_t* epoch;    // this sweep's epoch (k_flow_epoch)
-  uint32_t* err;
-  uint32_t* wave_ctr;       // [XCD]: waves started (cleared by k_flow_epoch)
-  uint32_t* done;           // [octant]: tasks done
-  uint32_t* mode;           // [octant]: 0 undecided, 1 static split, 2 claims
-  uint32_t* next;           // [octant]: tasks claimed (claims mode)
-  uint32_t waves;           // waves per octant
-  uint32_t barrier;         // polls a wave waits for its octant's W waves to arrive
+// The whole sweep of one source iteration in one launch.  A wave takes one
+// row of cells along x of one octant (a pencil: Geometry::pen) and updates
+// the octant's swept cells of it in order, for 64 velocities: the x upwind
+// values are its own last results, kept in registers, and the y and z ones
+// are other rows' results, read from the XCD's L2.  Rows, and with several
+// right-hand sides or more than 64 velocities per octant the (right-hand
+// side, 64 velocities) units of a row, are claimed from a counter per octant in
+// an order in which every row follows the rows it reads.  So the earliest
+// unfinished row can always proceed, whatever number of waves is resident,
+// and no wait is circular: the launch needs no residency and runs beside
+// other streams' kernels.
+//
+// A block sweeps the octant numbered like the XCD it runs on (its hardware
+// XCD id), so all producers and consumers of an octant's slots share one L2.
+// A row's progress is one word: the launch's base plus 1 + the oriented x of
+// its last finished task.  In a task's turn the wave issues the loads of what
+// comes next (the upwind values of the next task, if the rows (j -+ 1, k) and
+// (j, k -+ 1) are known to be past it, and the previous value of the task after
+// the next two, which waits for nothing), updates the task, waits until the
+// task before it has reached L2 and publishes that one.  A row so trails the
+// rows it reads by two to three tasks.  Progress is polled with agent-scope
+// loads, which miss the CU's L1; progress words and claim counters of two
+// octants share no cache line, or two XCDs would write it.  Values are plain
+// loads: no CU loads a slot's lines before they are final within the launch
+// (readers wait for the row's progress; the task's own read of the previous
+// value is followed by its store, which updates that CU's L1; slots are whole
+// cache lines, see Dims::vs), and the L1 starts the launch invalidated.
+// Every wait gives up after `spin` polls (a safety net: it sets err and the
+// wave ends, so the grid always drains); k_pencil_done then checks that every
+// octant's tasks were done.
+//
+// The update is sweep1_task's, operation for operation.  Where no axis is
+// first order (most tasks) the products of velocity and coefficient and the
+// denominator are the same for every task, so they stay in registers, and
+// the division is Markstein's: with r = 1 / den correctly rounded and q
+// refined twice by fma(fma(-den, q, num), r, q), the last step rounds
+// correctly (P. Markstein, IBM J. Res. Dev. 34, 1990); numerators whose
+// remainders could underflow take the division instead.  Same bits either way.
+//
+// What bounds it: at 200^3 the bytes between L2 and memory (rows are read again
+// for the next two diagonals; 11.5 ms where one read and one write of the
+// octants' slots take about 8.3 ms at a large copy's rate), at small images the
+// chain of rows, (Ny + Nz) hops of a few tasks each.  Sweep of one iteration,
+// one launch per hyperplane or per-cell flags before / rows: 32^3 pack, 27
+// velocities 0.54 / 0.20 ms, 45 x 38 x 41 0.46 / 0.30, sphere in 64^3 1.21 /
+// 0.84, 108 x 97 x 101 2.51 / 1.85, 96^3 with 216 velocities 16.1 / 6.0, 200^3
+// 16.5 / 11.5, six Kn in 112^3 16.3 / 10.3, 128^3 refined 8.7 / 2.9.  With the
+// octants' counters and words in shared lines: 32^3 0.24, 45 x 38 x 41 0.34,
+// 64^3 0.87.
+//
+// A re-poll of a row's progress waits 20 x 64 cycles: fewer polls in flight
+// leave the memory system to the rows being waited for.
+constexpr int kPenSleep = 20;
+
+template <typename T>
+struct PencilArgs {
+  T* f;
+  const T* fw;              // corner store [corner][octant][velocity]
+  double* part;             // [unit][octant][cell][4] partial moments; null = skip
+  uint32_t* prog;           // [unit][octant][row]: progress
+  uint32_t* st;             // the launch's state (k_pencil_begin)
   const double* cx;
   const double* cy;
   const double* cz;
   const double* w;
-  const SweepCoef* coef;
-  const double* fw;         // corner store [corner][octant][velocity]
-  double mu0;
-  int64_t off[9];           // first task of each octant in rec
-  int64_t ostride;          // elements of f per octant
-  int64_t nslot;            // flags per octant (stored slots + the zero slot)
+  const double* mu;         // per right-hand side
+  int64_t ostride, rs_f, rs_fw, rs_mom;
+  uint32_t off[9];          // first row of each octant in the row list
+  uint32_t vs, vs_fw;       // velocities per slot of f (padded), of fw
+  uint32_t Nc8, chunks;     // velocities, units of 64 velocities
+  uint32_t units, group;    // units; units taken together, row by row
+  uint32_t Nx, Ny, npen;    // rows of the grid: Ny, progress words per octant (pencil_words)
+  double c0, c1, c2, d1;    // 1.5/ds, 2/ds, -0.5/ds, 1/ds
+  const TaskRec* rec;           // Geometry::pen_rec
+  const Geometry::Pencil* pens; // Geometry::pen
+  const Mom* mom;
   uint32_t spin;            // polls before a wait gives up
-  uint32_t probe;           // nonzero: residency probe only (flow_setup), this many polls
-  uint32_t* diag;           // [block]: XCD id, then [grid + block]: tasks done
+  // defect correction (kDC, see SweepArgs)
+  float* dc_r;
+  const float* dc_e;
+  int32_t dc_fold, dc_first;
 };
 
-// Next epoch of the flags; the counters of the launch cleared.  st: [0]
-// epoch, [1..6] err, [8..15] waves started per XCD, [16..23] tasks done per
-// octant, [24] the residency probe's count, [32..39] mode per octant,
-// [40..47] tasks claimed per octant.
-__global__ void k_flow_epoch(uint32_t* st) {
-  if (threadIdx.x == 0) __hip_atomic_fetch_add(st, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (threadIdx.x < 56) st[8 + threadIdx.x] = 0u;
+// Records read past the last row's end (never used).
+constexpr size_t kPenPad = 4;
+
+// State words of the pencil sweep: [0] the launch's progress base, [1..6]
+// err, [kPenOct * (1 + octant)] a line per octant, as only its XCD writes it
+// during the sweep: rows claimed, tasks done.
+constexpr int kPenDone = 1, kPenNext = 0, kPenOct = 32, kPenState = 9 * kPenOct;
+static_assert(kPenErrWords == 6, "st[1..6]");
+
+// Next progress base; the counters of the launch cleared.
+__global__ void k_pencil_begin(uint32_t* st, uint32_t step) {
+  if (threadIdx.x == 0) __hip_atomic_fetch_add(st, step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x < 8) {
+    uint32_t* const q = st + kPenOct * (1 + threadIdx.x);
+    q[kPenNext] = q[kPenDone] = 0u;
+  }
 }
 
 // After the sweep: every octant's tasks done (else err, unless already set).
-struct FlowCounts {
+struct PencilCounts {
   uint32_t n[8];
 };
-__global__ void k_flow_done(uint32_t* st, FlowCounts c) {
+__global__ void k_pencil_done(uint32_t* st, PencilCounts c) {
   const uint32_t o = threadIdx.x;
-  if (o < 8 && st[16 + o] != c.n[o] &&
+  const uint32_t done = o < 8 ? st[kPenOct * (1 + o) + kPenDone] : 0u;
+  if (o < 8 && done != c.n[o] &&
       __hip_atomic_fetch_add(st + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) {
     st[2] = o;
-    st[3] = st[16 + o];
-    st[4] = 0xffffffffu;
-    st[5] = c.n[o];
+    st[3] = done;
+    st[4] = c.n[o];
+    st[5] = 0xffffffffu;
   }
 }
 
-// XCD of every block of a grid of n one-wave blocks (flow_probe)
-__global__ void k_flow_probe(uint32_t* out, uint32_t n) {
+// XCD of every block of a grid of n one-wave blocks.
+__global__ void k_xcd_probe(uint32_t* out, uint32_t n) {
   if (threadIdx.x == 0 && blockIdx.x < n) out[blockIdx.x] = __builtin_amdgcn_s_getreg((3 << 11) | 20) & 15u;
 }
 
-// What a task needs before its upwind values: its record's fields, the
-// cell's moments, the slot's previous value and one poll of the flags it
-// waits for (one per axis at most; an axis without a wait
-// issues no load and reads as ep).
-struct FlowTask {
-  uint32_t self, cell, flg;
-  uint32_t nbs[6];          // the record's source words
-  const uint32_t* wt[3];
-  uint32_t v[3];
-  Mom m;
-  double fp;
-};
-
 // An agent-scope load (it misses the CU's L1); the caller makes it uniform
 // where it compares, so that several polls go out before the first returns.
-__device__ __forceinline__ uint32_t flow_poll(const uint32_t* p) {
+__device__ __forceinline__ uint32_t pencil_poll(const uint32_t* p) {
   return __hip_atomic_load(const_cast<uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// One poll of each flag the task waits for.
-__device__ __forceinline__ void flow_poll3(FlowTask& t, uint32_t ep) {
-#pragma unroll
-  for (int ax = 0; ax < 3; ++ax) t.v[ax] = t.wt[ax] ? flow_poll(t.wt[ax]) : ep;
+// num / den with r = 1 / den correctly rounded (see above): correctly
+// rounded for |num| in [2^-800, 2^800) and den in [2^-100, 2^100].
+__device__ __forceinline__ double markstein_div(double num, double den, double r) {
+  double q = num * r;
+  q = __builtin_fma(__builtin_fma(-den, q, num), r, q);
+  return __builtin_fma(__builtin_fma(-den, q, num), r, q);
+}
+// Wait until at most N vector memory operations are outstanding: the builtin,
+// so that the compiler's own count of them stays exact, between fences that
+// keep its loads and stores on their side.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | (N >> 4) << 14);
+  asm volatile("" ::: "memory");
 }
 
-// The flags a task waits for, from its record, and one poll of each.
-__device__ __forceinline__ void flow_targets(FlowTask& t, const TaskRec& r, const uint32_t* flo, uint32_t ep) {
-#pragma unroll
-  for (int ax = 0; ax < 3; ++ax) {
-    const uint32_t w1 = (uint32_t)r.w[1 + 2 * ax], w2 = (uint32_t)r.w[2 + 2 * ax];
-    t.wt[ax] = (w1 >> 28) == 8u   ? flo + (w1 & 0x0fffffffu)
-               : (w2 >> 28) == 8u ? flo + (w2 & 0x0fffffffu)
-                                  : nullptr;
-  }
-  flow_poll3(t, ep);
+// The exponent of v, from 0 to kMidSpan - 1 where |v| is in [2^-800, 2^800).
+constexpr uint32_t kMidSpan = 1600u;
+__device__ __forceinline__ uint32_t mid_exponent(double v) {
+  return ((uint32_t)(__builtin_bit_cast(uint64_t, v) >> 52) & 0x7ffu) - (1023u - 800u);
 }
 
-// The rest of a task's set-up: record fields, moments, previous value.
-__device__ __forceinline__ void flow_fields(FlowTask& t, const TaskRec& r, const Mom* __restrict__ mom,
-                                            const double* fo, int lane) {
-  t.self = (uint32_t)r.w[0] & 0x0fffffffu;
-  t.cell = (uint32_t)r.w[7] & 0x0fffffffu;
-  t.flg = (uint32_t)r.w[7] >> 28;
-#pragma unroll
-  for (int q = 0; q < 6; ++q) t.nbs[q] = (uint32_t)r.w[1 + q];
-  t.m = ld_const(mom + t.cell);
-  t.fp = fo[(size_t)t.self * 64 + lane];
-}
+// The two halves of a row task's record (Geometry::pen_rec).
+struct alignas(8) PenOwn {
+  uint32_t w0, w1;
+};
+struct alignas(8) PenNbr {
+  uint32_t nb[4], x[2];
+};
 
-__device__ __forceinline__ void flow_issue(FlowTask& t, const TaskRec& r, const Mom* __restrict__ mom,
-                                           const double* fo, const uint32_t* flo, int lane, uint32_t ep) {
-  t.self = (uint32_t)r.w[0] & 0x0fffffffu;
-  t.cell = (uint32_t)r.w[7] & 0x0fffffffu;
-  t.flg = (uint32_t)r.w[7] >> 28;
-#pragma unroll
-  for (int q = 0; q < 6; ++q) t.nbs[q] = (uint32_t)r.w[1 + q];
-#pragma unroll
-  for (int ax = 0; ax < 3; ++ax) {
-    const uint32_t w1 = t.nbs[2 * ax], w2 = t.nbs[2 * ax + 1];
-    t.wt[ax] = (w1 >> 28) == 8u   ? flo + (w1 & 0x0fffffffu)
-               : (w2 >> 28) == 8u ? flo + (w2 & 0x0fffffffu)
-                                  : nullptr;
-  }
-  t.m = ld_const(mom + t.cell);
-  t.fp = fo[(size_t)t.self * 64 + lane];
-  flow_poll3(t, ep);
-}
-
-// Whether the polls read the sweep's epoch on every flag the task waits for.
-__device__ __forceinline__ bool flow_ready(const FlowTask& t, uint32_t ep) {
-  return __builtin_amdgcn_readfirstlane(t.v[0]) == ep && __builtin_amdgcn_readfirstlane(t.v[1]) == ep &&
-         __builtin_amdgcn_readfirstlane(t.v[2]) == ep;
-}
-
-// The first velocity of an upwind source word of a flow record: bits 0..27
-// an index, bits 28..30 x, bit 31 c.  c = 0: slot of octant o ^ x; c = 1,
-// x = 0: slot of octant o, whose flag the task waits for; c = 1, x != 0:
-// corner store entry (corner * 8 + octant).  The host resolves the reads
-// of wall slots the reference switched (switched_source) into the second and
-// third forms, so the sweep reads every source through this one path.
-__device__ __forceinline__ const double* flow_source(const FlowArgs& a, uint32_t o, uint32_t wq) {
-  const uint32_t x = (wq >> 28) & 7u;
-  const size_t idx = (size_t)(wq & 0x0fffffffu) * 64;
-  return (wq >> 31) && x ? a.fw + idx : a.f + (size_t)(o ^ x) * a.ostride + idx;
-}
-
-// Claim the octant's next task (lane 0's value; the caller makes it uniform
-// where it uses it, so that the claim overlaps other loads).
-__device__ __forceinline__ uint32_t flow_claim(uint32_t* next, int lane) {
-  uint32_t v = 0;
-  if (lane == 0) v = __hip_atomic_fetch_add(next, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  return v;
-}
-
-// Set the octant's mode to m unless it is set: the mode that holds.
-__device__ __forceinline__ uint32_t flow_decide(uint32_t* mode, uint32_t m, int lane) {
-  uint32_t old = 0;
-  if (lane == 0)
-    __hip_atomic_compare_exchange_strong(mode, &old, m, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  old = __builtin_amdgcn_readfirstlane(old);
-  return old ? old : m;
-}
-
-// Poll until the three flags read ep (false: gave up, or another wave did).
-// A wave that gives up records err = 1 and the octant, task, slot, epoch and
-// last value it saw in err[1..5] for the host's message.
-__device__ __forceinline__ bool flow_wait(FlowTask& t, uint32_t ep, uint32_t* err, uint32_t spin, uint32_t o,
-                                          uint32_t k, const uint32_t* flo) {
-  for (uint32_t it = 0; it < spin; ++it) {
-    const uint32_t v0 = __builtin_amdgcn_readfirstlane(t.v[0]), v1 = __builtin_amdgcn_readfirstlane(t.v[1]),
-                   v2 = __builtin_amdgcn_readfirstlane(t.v[2]);
-    if (v0 == ep && v1 == ep && v2 == ep) return true;
-    if ((it & 63u) == 63u && __builtin_amdgcn_readfirstlane(flow_poll(err)) != 0u) return false;
-    // a re-poll waits 16 x 64 cycles: fewer polls in flight leave the memory
-    // system to the stores being waited for (40^3 pack, sweep ms for a wait
-    // of 1, 2, 4, 8, 16: 0.593, 0.542, 0.490, 0.452, 0.434; 200^3 unchanged)
-    __builtin_amdgcn_s_sleep(16);
-    flow_poll3(t, ep);
-  }
-  if (threadIdx.x == 0) {
-    const bool b0 = t.v[0] != ep, b1 = t.v[1] != ep;
-    err[1] = o;
-    err[2] = k;
-    const uintptr_t p0 = (uintptr_t)t.wt[0], p1 = (uintptr_t)t.wt[1], p2 = (uintptr_t)t.wt[2];
-    err[3] = (uint32_t)(((b0 ? p0 : b1 ? p1 : p2) - (uintptr_t)flo) / sizeof(uint32_t));
-    err[4] = ep;
-    err[5] = b0 ? t.v[0] : b1 ? t.v[1] : t.v[2];
-    __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  return false;
-}
-
-// One wave: its tasks of its XCD's octant (k = w, w + W, ... or claimed),
-// pipelined so that a task costs one memory round trip besides its update:
-// the next task's flags are polled while this task computes, and after this
-// task's stores its moments, previous value and, if those flags were set,
-// its upwind values go out before the wait for the stores.  This task's
-// flag is set before any poll of the next task is looked at again, so a wave
-// never waits for its own task.
-// The records, moments and coefficients, which nothing in the launch writes,
-// come through restrict arguments, so their loads are scalar loads and the
-// kernel runs 6 waves per SIMD (SGPR-bound; its occupancy query says 7).
-template <bool kEarly>
-__global__ __launch_bounds__(64) void k_sweep_flow(FlowArgs a, const TaskRec* __restrict__ rec,
-                                                   const Mom* __restrict__ mom, const SweepCoef* __restrict__ coef) {
+template <typename T, int kDC>
+__global__ __launch_bounds__(64) void k_sweep_pencil(PencilArgs<T> args) {
+  // Arguments are read where they are used (args_now), not held in registers
+  // across the row loop: the row loop's own scalars fill the SGPRs.
+  (void)args;
+#if defined(__HIP_DEVICE_COMPILE__)
+  using ArgsPtr = const __attribute__((address_space(4))) PencilArgs<T>*;
+  auto args_now = []() -> ArgsPtr {
+    ArgsPtr p = (ArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+  };
+#else
+  auto args_now = [&]() { return &args; };
+#endif
   const int lane = threadIdx.x;
-  if (a.probe) {  // are all blocks of this grid resident at once?  (st[24] counts them in)
-    if (lane == 0) __hip_atomic_fetch_add(a.done + 8, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t seen = 0;
-    for (uint32_t it = 0; it < a.probe; ++it) {
-      seen = __builtin_amdgcn_readfirstlane(flow_poll(a.done + 8));
-      if (seen >= gridDim.x) break;
-      __builtin_amdgcn_s_sleep(2);
-    }
-    if (lane == 0) a.diag[blockIdx.x] = seen >= gridDim.x ? 0xffffffffu : seen;
-    return;
-  }
   const uint32_t o = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 7u);
-  uint32_t tk = 0;
-  if (lane == 0) tk = __hip_atomic_fetch_add(a.wave_ctr + o, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint32_t wv = __builtin_amdgcn_readfirstlane(tk);
-  if (lane == 0) a.diag[blockIdx.x] = o;
-  // the octant's mode: the static split once its W waves have all arrived
-  // (the W-th arrival sets it), claims if a wave waited `barrier` polls first
-  uint32_t md = wv + 1 == a.waves ? flow_decide(a.mode + o, 1u, lane) : 0u;
-  for (uint32_t it = 0; md == 0u && it < a.barrier; ++it) {
-    md = __builtin_amdgcn_readfirstlane(flow_poll(a.mode + o));
-    if (md == 0u) __builtin_amdgcn_s_sleep(2);
+  uint32_t np, total;
+  uint32_t* st;
+  {
+    const auto a = args_now();
+    np = a->off[o + 1] - a->off[o];
+    total = np * a->units;
+    st = a->st;
   }
-  if (md == 0u) md = flow_decide(a.mode + o, 2u, lane);
-  const bool claims = md == 2u;
-  const int64_t base = a.off[o], n = a.off[o + 1] - base;
-  // the epoch through the vector path (an agent-scope load): a scalar load
-  // could be served by a scalar cache line of the previous kernel
-  const uint32_t ep = __builtin_amdgcn_readfirstlane(flow_poll(a.epoch));
-  double* const fo = a.f + (size_t)o * a.ostride;
-  uint32_t* const flo = a.flags + (size_t)o * a.nslot;
+  auto claim = [&]() -> uint32_t {
+    uint32_t v = 0;
+    if (lane == 0) v = __hip_atomic_fetch_add(st + kPenOct * (1 + o) + kPenNext, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return v;
+  };
+  // the progress base through the vector path (an agent-scope load): a scalar
+  // load could be served by a scalar cache line of the previous kernel
+  uint32_t cl = claim();
+  const uint32_t base = __builtin_amdgcn_readfirstlane(pencil_poll(st));
   uint32_t done = 0;
-  // the lane's velocity, the same for every task of the wave (64 per octant)
-  const double cxl = a.cx[lane], cyl = a.cy[lane], czl = a.cz[lane], wl = a.w[lane];
-  const bool px = osx((int)o) > 0, py = osy((int)o) > 0, pz = osz((int)o) > 0;
-  uint32_t* const next = a.next + o;
-  if constexpr (!kEarly) {
-  // static: tasks wv, wv + W, ... (a wave beyond W has none); claims: the
-  // next unclaimed task, claimed one task ahead
-  int64_t k = claims ? (int64_t)__builtin_amdgcn_readfirstlane(flow_claim(next, lane)) : wv < a.waves ? wv : n;
-  if (k < n) {
-    FlowTask t;
-    flow_issue(t, ld_const(rec + base + k), mom, fo, flo, lane, ep);
-    int64_t kn = claims ? (int64_t)__builtin_amdgcn_readfirstlane(flow_claim(next, lane)) : k + a.waves;
-    TaskRec rn = ld_const(rec + base + (kn < n ? kn : k));
-    while (true) {
-      if (!flow_wait(t, ep, a.err, a.spin, o, (uint32_t)k, flo)) break;
-      asm volatile("" ::: "memory");  // the upwind loads stay after the polls that cleared them
-      double nb[6];
-#pragma unroll
-      for (int q = 0; q < 6; ++q) nb[q] = flow_source(a, o, t.nbs[q])[lane];
-      // the coefficients (eight entries, cache-resident) with the upwind values
-      const SweepCoef cf = ld_const(coef + (t.flg & 7u));
-      // sweep1_task's update, operation for operation
-      const double mx = px ? t.m.x : -t.m.x;
-      const double my = py ? t.m.y : -t.m.y;
-      const double mz = pz ? t.m.z : -t.m.z;
-      double tt = cxl * mx;
-      tt = tt + cyl * my;
-      tt = tt + czl * mz;
-      const double feq = wl * (t.m.r + 1.0 * tt);
-      double num = a.mu0 * (feq - 0.5 * t.fp);
-      num = num + cxl * cf.x1 * nb[0];
-      num = num + cxl * cf.x2 * nb[1];
-      num = num + cyl * cf.y1 * nb[2];
-      num = num + cyl * cf.y2 * nb[3];
-      num = num + czl * cf.z1 * nb[4];
-      num = num + czl * cf.z2 * nb[5];
-      double den = 0.5 * a.mu0 + cxl * cf.dx;
-      den = den + cyl * cf.dy;
-      den = den + czl * cf.dz;
-      const double fnew = num / den;
-      const uint32_t self = t.self, cell = t.cell;
-      fo[(size_t)self * 64 + lane] = fnew;
-      if (a.part) {
-        const double z = wave_sum4(fnew, cxl * fnew, cyl * fnew, czl * fnew);
-        if ((lane & 15) == 0) {
-          const uint32_t q = (uint32_t)lane >> 4;
-          const double zz = ((kOctNeg >> (4 * o + q)) & 1u) ? -z : z;
-          a.part[((size_t)cell * 8 + o) * 4 + q] = zz;
-        }
-      }
-      const bool more = kn < n;
-      uint32_t knn = 0;
-      if (more) {
-        flow_issue(t, rn, mom, fo, flo, lane, ep);
-        if (claims) knn = flow_claim(next, lane);
-      }
-      // the slot's values (and partials) reach L2 before its flag
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-      if (lane == 0) __hip_atomic_store(flo + self, ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      ++done;
-      if (!more) break;
-      k = kn;
-      kn = claims ? (int64_t)__builtin_amdgcn_readfirstlane(knn) : kn + a.waves;
-      rn = ld_const(rec + base + (kn < n ? kn : k));
+  uint32_t c = __builtin_amdgcn_readfirstlane(cl);
+  // byte offsets of the lane: its velocity in a slot (loads; stores, where
+  // idle lanes are out of the buffer's range), its partial moment (lanes 0,
+  // 16, 32, 48; the others out of range)
+  constexpr uint32_t kOut = 0xf0000000u;
+  const uint32_t voff_p = (lane & 15) == 0 ? (uint32_t)(lane >> 4) * 8u : kOut;
+  uint32_t unit = 0xffffffffu, voff = 0, voff_st = 0;
+  // the unit's constants: signed velocities (the octant's signs), weight, and
+  // the products of a second-order task
+  double scx = 0, scy = 0, scz = 0, wl = 0, mu = 0;
+  double ax1 = 0, ax2 = 0, ay1 = 0, ay2 = 0, az1 = 0, az2 = 0, den0 = 1, rden0 = 1;
+  uint32_t mid = 0;  // numerator exponents the fast division takes (0: none)
+  while (c < total) {
+    const auto a = args_now();
+    const uint32_t units = a->units, group = a->group, chunks = a->chunks;
+    const uint32_t gsz = np * group, gr = c / gsz, cr = c - gr * gsz;
+    const uint32_t gn = min(group, units - gr * group);
+    const uint32_t p = cr / gn, u = gr * group + (cr - p * gn);
+    const uint32_t rhs = u / chunks, ch = u - rhs * chunks;
+    const double d1 = a->d1, c0 = a->c0, c1 = a->c1, c2 = a->c2;
+    if (u != unit) {
+      unit = u;
+      const uint32_t l = ch * 64u + (uint32_t)lane;
+      const bool lact = l < a->Nc8;
+      const uint32_t ll = lact ? l : ch * 64u;  // idle lanes stay in the unit's own lines
+      voff = ll * (uint32_t)sizeof(T);
+      voff_st = lact ? voff : kOut;
+      const double cxl = a->cx[ll], cyl = a->cy[ll], czl = a->cz[ll];
+      wl = a->w[ll];
+      mu = *const_ptr(a->mu + rhs);
+      scx = osx((int)o) > 0 ? cxl : -cxl;
+      scy = osy((int)o) > 0 ? cyl : -cyl;
+      scz = osz((int)o) > 0 ? czl : -czl;
+      ax1 = cxl * c1;
+      ax2 = cxl * c2;
+      ay1 = cyl * c1;
+      ay2 = cyl * c2;
+      az1 = czl * c1;
+      az2 = czl * c2;
+      den0 = 0.5 * mu + cxl * c0;
+      den0 = den0 + cyl * c0;
+      den0 = den0 + czl * c0;
+      rden0 = 1.0 / den0;
+      mid = __builtin_amdgcn_ballot_w64(!(den0 >= 0x1p-100 && den0 <= 0x1p100)) == 0 ? kMidSpan : 0u;
     }
-  }
-  } else {
-  // static: tasks wv, wv + W, ... (a wave beyond W has none); claims: the
-  // next unclaimed task
-  int64_t k = claims ? (int64_t)__builtin_amdgcn_readfirstlane(flow_claim(next, lane)) : wv < a.waves ? wv : n;
-  if (k < n) {
-    // task k: its record's fields, moments, previous value and upwind values
-    FlowTask t;
-    flow_issue(t, ld_const(rec + base + k), mom, fo, flo, lane, ep);
-    if (!flow_wait(t, ep, a.err, a.spin, o, (uint32_t)k, flo)) goto out;
-    asm volatile("" ::: "memory");  // the upwind loads stay after the polls that cleared them
-    double nb[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) nb[q] = flow_source(a, o, t.nbs[q])[lane];
-    int64_t kn = claims ? (int64_t)__builtin_amdgcn_readfirstlane(flow_claim(next, lane)) : k + a.waves;
-    TaskRec rn = ld_const(rec + base + (kn < n ? kn : k));
-    while (true) {
-      const bool more = kn < n;
-      // the next task's flags, polled while this task computes
-      FlowTask tn;
-      if (more) flow_targets(tn, rn, flo, ep);
-      // the coefficients (eight entries, cache-resident)
-      const SweepCoef cf = ld_const(coef + (t.flg & 7u));
-      // sweep1_task's update, operation for operation
-      const double mx = px ? t.m.x : -t.m.x;
-      const double my = py ? t.m.y : -t.m.y;
-      const double mz = pz ? t.m.z : -t.m.z;
-      double tt = cxl * mx;
-      tt = tt + cyl * my;
-      tt = tt + czl * mz;
-      const double feq = wl * (t.m.r + 1.0 * tt);
-      double num = a.mu0 * (feq - 0.5 * t.fp);
-      num = num + cxl * cf.x1 * nb[0];
-      num = num + cxl * cf.x2 * nb[1];
-      num = num + cyl * cf.y1 * nb[2];
-      num = num + cyl * cf.y2 * nb[3];
-      num = num + czl * cf.z1 * nb[4];
-      num = num + czl * cf.z2 * nb[5];
-      double den = 0.5 * a.mu0 + cxl * cf.dx;
-      den = den + cyl * cf.dy;
-      den = den + czl * cf.dz;
-      const double fnew = num / den;
-      // the next task's polls, read before this task's stores go out (a
-      // wait on them after the stores would wait for the stores too)
-      const bool early = more && flow_ready(tn, ep);
-      const uint32_t self = t.self, cell = t.cell;
-      fo[(size_t)self * 64 + lane] = fnew;
-      if (a.part) {
-        const double z = wave_sum4(fnew, cxl * fnew, cyl * fnew, czl * fnew);
-        if ((lane & 15) == 0) {
-          const uint32_t q = (uint32_t)lane >> 4;
-          const double zz = ((kOctNeg >> (4 * o + q)) & 1u) ? -z : z;
-          a.part[((size_t)cell * 8 + o) * 4 + q] = zz;
-        }
-      }
-      // the next task's loads go out with this task's stores: its upwind
-      // values too when its flags were already set (it then needs no memory
-      // round trip of its own before its update)
-      uint32_t knn = 0;
-      if (more) {
-        flow_fields(tn, rn, mom, fo, lane);
-        if (early) {
-          asm volatile("" ::: "memory");  // the upwind loads stay after the polls that cleared them
-#pragma unroll
-          for (int q = 0; q < 6; ++q) nb[q] = flow_source(a, o, tn.nbs[q])[lane];
-        }
-        if (claims) knn = flow_claim(next, lane);
-        else rn = ld_const(rec + base + (kn + a.waves < n ? kn + a.waves : kn));
-      }
-      // the slot's values (and partials) reach L2 before its flag
-      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-      if (lane == 0) __hip_atomic_store(flo + self, ep, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      ++done;
-      if (!more) break;
-      t = tn;
-      k = kn;
-      if (claims) {
-        kn = (int64_t)__builtin_amdgcn_readfirstlane(knn);
-        rn = ld_const(rec + base + (kn < n ? kn : k));
+    const Geometry::Pencil pen = *const_ptr(a->pens + a->off[o] + p);
+    const uint32_t n = pen.n & 0x3fffffffu, vs = a->vs;
+    const int64_t rs_mom = a->rs_mom;
+    const size_t fbase = (size_t)rhs * a->rs_f + (size_t)o * a->ostride + (size_t)pen.lo * vs;
+    // the row's window of f, and of the correction and the residual
+    T* const fwin = a->f + fbase;
+    const int fbytes = (int)(pen.len * vs * (uint32_t)sizeof(T));
+    float* const ewin = kDC == 1 ? const_cast<float*>(a->dc_e) + fbase : nullptr;
+    float* const rwin = kDC != 0 ? a->dc_r + fbase : nullptr;
+    const bool dc_flag = kDC == 1 ? a->dc_fold != 0 : kDC == 2 ? a->dc_first != 0 : false;
+    const ConstPtr<Mom> momr = const_ptr(a->mom + (size_t)rhs * rs_mom + pen.cell);
+    const bool has_part = a->part != nullptr;  // else the partials' stores are out of range
+    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
+        has_part ? a->part + (((size_t)u * 8 + o) * rs_mom + pen.cell) * 4 : nullptr, 0,
+        has_part ? (int)(a->Nx + 2u) * 32 : 0, kBufferWord3);
+    uint32_t* const own = a->prog + ((size_t)u * 8 + o) * a->npen + pen.id;
+    const int32_t sy = osy((int)o), sz = osz((int)o) * (int32_t)a->Ny;
+    const ConstPtr<TaskRec> rr = const_ptr(a->rec + pen.rec);
+    const uint32_t last = n - 1u;
+    const bool hasy = pen.n >> 31, hasz = (pen.n >> 30) & 1u;
+    // The neighbour rows' progress as last seen (lim: the smaller; past the
+    // row's end where there is no neighbour or it is finished).  Lane 0 polls
+    // the y neighbour's, lane 1 the z neighbour's, the others the row's own.
+    constexpr int32_t kAll = 0x3fffffff;
+    int32_t py = hasy ? 0 : kAll, pz = hasz ? 0 : kAll, lim = min(py, pz);
+    const int32_t pofs = lane == 0 ? -sy : lane == 1 ? -sz : 0;
+    const int32_t Nx = (int32_t)a->Nx;
+    auto poll = [&]() -> uint32_t { return pencil_poll(own + pofs); };
+    auto polled = [&](uint32_t v) {
+      const int32_t vy = (int32_t)((uint32_t)__builtin_amdgcn_readlane((int)v, 0) - base);
+      const int32_t vz = (int32_t)((uint32_t)__builtin_amdgcn_readlane((int)v, 1) - base);
+      py = hasy && vy <= Nx ? vy : kAll;
+      pz = hasz && vz <= Nx ? vz : kAll;
+      lim = min(py, pz);
+    };
+    auto ox1 = [](uint32_t w1) -> int32_t { return (int32_t)((w1 >> 14) & 0x3fffu); };
+    auto publish = [&](uint32_t v) {
+      // every lane writes the same word
+      __hip_atomic_store(own, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    };
+    bool alive = true;
+    // What a task's loads leave: Own three tasks ahead (its slot's previous
+    // value, which waits for no other row), Nbr one task ahead (the upwind
+    // values, once the rows they come from are done).
+    struct Own {
+      T fp;
+      float fe;
+      uint32_t w0, w1;      // the record's
+    };
+    struct Nbr {
+      T nb[4], xl1, xl2;
+      Mom m;
+      int bytes;            // 0: not loaded
+    };
+    constexpr int kSelf = sizeof(T) == 8 ? 3 : 2;
+    // byte offset of a source word (in 8-byte elements)
+    auto src_off = [](uint32_t w) -> uint32_t { return sizeof(T) == 8 ? w : w >> 1; };
+    auto self_off = [](uint32_t w0) -> uint32_t { return (w0 & 0x0fffffffu) << kSelf; };
+    auto mom_off = [](uint32_t w1) -> uint32_t { return (w1 & 0x3fffu) << 5; };
+    auto ld_mom = [&](uint32_t w1) -> Mom {
+      return *(ConstPtr<Mom>)((ConstPtr<char>)momr + mom_off(w1));
+    };
+    // One load (two or three with defect correction); t past the row: the same
+    // from an empty buffer (no traffic).
+    auto issue_own = [&](Own& s, const PenOwn& r, uint32_t t) __attribute__((always_inline)) {
+      const int bytes = t < n ? fbytes : 0;
+      s.w0 = r.w0;
+      s.w1 = r.w1;
+      const uint32_t so = self_off(r.w0);
+      if constexpr (kDC == 1)
+        s.fe = buf_load<float>(__builtin_amdgcn_make_buffer_rsrc(ewin, 0, dc_flag ? bytes >> 1 : 0, kBufferWord3), voff >> 1, so >> 1);
+      if constexpr (kDC == 2)
+        s.fe = buf_load<float>(__builtin_amdgcn_make_buffer_rsrc(rwin, 0, bytes, kBufferWord3), voff, so);
+      s.fp = buf_load<T>(__builtin_amdgcn_make_buffer_rsrc(fwin, 0, bytes, kBufferWord3), voff, so);
+    };
+    // Four loads, more where a run starts or a wall slot was switched; bytes 0:
+    // the four from an empty buffer.
+    auto issue_nb = [&](Nbr& s, const PenNbr& r, uint32_t w0, uint32_t w1, int bytes) __attribute__((always_inline)) {
+      s.bytes = bytes;
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(fwin, 0, bytes, kBufferWord3);
+      if (!(w1 & Geometry::kPenX1Reg)) {
+        s.xl1 = buf_load<T>(rs, voff, src_off(r.x[0]));
+        s.xl2 = buf_load<T>(rs, voff, src_off(r.x[1] & ~7u));
       } else {
-        kn += a.waves;
+        asm volatile("" : "=v"(s.xl1), "=v"(s.xl2));  // not read: no copies where the paths meet
       }
-      if (!early) {  // the next task waits on this one's or others' flags
-        if (!flow_wait(t, ep, a.err, a.spin, o, (uint32_t)k, flo)) break;
-        asm volatile("" ::: "memory");  // the upwind loads stay after the polls that cleared them
+      // far words are beyond every window: these loads return 0 for them
 #pragma unroll
-        for (int q = 0; q < 6; ++q) nb[q] = flow_source(a, o, t.nbs[q])[lane];
+      for (int q = 0; q < 4; ++q) s.nb[q] = buf_load<T>(rs, voff, src_off(r.nb[q]));
+      if (w0 >> 31 && bytes != 0) {
+        const auto b = args_now();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t w = r.nb[q];
+          if (w & Geometry::kPenFar) {
+            const size_t row = w & 0x3fffffffu;
+            const T* src = (w & Geometry::kPenFw) ? b->fw + (size_t)rhs * b->rs_fw + row * b->vs_fw
+                                                  : b->f + (size_t)rhs * b->rs_f + row * b->vs;
+            s.nb[q] = *reinterpret_cast<const T*>(reinterpret_cast<const char*>(src) + voff);
+          }
+        }
+      }
+    };
+    double h1 = 0, h2 = 0;         // x upwind values
+    uint32_t k = 0;
+    uint32_t pub = base;                // progress up to task k - 1
+    PenOwn ro;                          // the next records to load, own and upwind part
+    PenNbr rn;
+    constexpr uint32_t kFarWait = Geometry::kPenWaitY2 | Geometry::kPenWaitZ2;
+    auto rec_own = [&](uint32_t t) -> PenOwn { return *(ConstPtr<PenOwn>)(rr + t); };
+    auto rec_nbr = [&](uint32_t t) -> PenNbr { return *(ConstPtr<PenNbr>)((ConstPtr<char>)(rr + t) + sizeof(PenOwn)); };
+    // Task k, loaded in oc and nc: before its update the upwind values of task
+    // k + 1 (its own part in o1) go into nn if its rows are done, and the own
+    // part of task k + 3 into o3.  Rows are taken as done by the smaller
+    // progress alone: a task that waits on one of them only, or on a row at
+    // distance 2, may be left to the loop's top.
+    auto turn = [&](Own& oc, Nbr& nc, Own& o1, Nbr& nn, Own& o3) __attribute__((always_inline)) {
+      const int32_t x1 = ox1(o1.w1);
+      int bytes = lim >= x1 && k + 1u < n ? fbytes : 0;
+      if (o1.w0 >> 31 && rn.x[1] & kFarWait) bytes = 0;
+      // the rows' progress is read again when the next task comes near it
+      const bool want = lim < x1 + 6;
+      asm volatile("" ::: "memory");  // the loads stay after the polls that cleared them
+      issue_nb(nn, rn, o1.w0, o1.w1, bytes);
+      issue_own(o3, ro, k + 3u);
+      uint32_t pv;
+      if (want) pv = poll();
+      ro = rec_own(k + 4u);
+      rn = rec_nbr(k + 2u);
+      nn.m = ld_mom(o1.w1);
+      if (!(oc.w1 & Geometry::kPenX1Reg)) {
+        asm volatile("" : "+v"(nc.xl1));  // a branch: runs start seldom
+        h2 = (oc.w1 & Geometry::kPenX2Reg) ? h1 : (double)nc.xl2;
+        h1 = (double)nc.xl1;
+      }
+      double fpv = (double)oc.fp;
+      if constexpr (kDC == 1) {
+        if (dc_flag) fpv = fpv + (double)oc.fe;
+      }
+      if constexpr (kDC == 2) fpv = dc_flag ? (double)oc.fe : fpv + (double)oc.fe;
+      // sweep1_task's update, operation for operation
+      double tt = scx * nc.m.x;
+      tt = tt + scy * nc.m.y;
+      tt = tt + scz * nc.m.z;
+      const double feq = wl * (nc.m.r + 1.0 * tt);
+      double num = mu * (feq - 0.5 * fpv);
+      double fnew, den = den0;
+      bool divide = true;
+      if ((oc.w0 & 0x70000000u) == 0u) {
+        num = num + ax1 * h1;
+        num = num + ax2 * h2;
+        num = num + ay1 * (double)nc.nb[0];
+        num = num + ay2 * (double)nc.nb[1];
+        num = num + az1 * (double)nc.nb[2];
+        num = num + az2 * (double)nc.nb[3];
+        divide = __builtin_amdgcn_ballot_w64(mid_exponent(num) >= mid) != 0;
+        fnew = markstein_div(num, den0, rden0);
+      } else {
+        // the axis' coefficients, selected on the scalar unit (opaque copies,
+        // so that the products are not kept in registers across tasks)
+        double k0 = c0, k1 = c1, k2 = c2, kd = d1;
+        asm volatile("" : "+s"(k0), "+s"(k1), "+s"(k2), "+s"(kd));
+        const bool fx = oc.w0 & 0x10000000u, fy = oc.w0 & 0x20000000u, fz = oc.w0 & 0x40000000u;
+        const double cxl = __builtin_fabs(scx), cyl = __builtin_fabs(scy), czl = __builtin_fabs(scz);
+        num = num + cxl * (fx ? kd : k1) * h1;
+        num = num + cxl * (fx ? 0.0 : k2) * h2;
+        num = num + cyl * (fy ? kd : k1) * (double)nc.nb[0];
+        num = num + cyl * (fy ? 0.0 : k2) * (double)nc.nb[1];
+        num = num + czl * (fz ? kd : k1) * (double)nc.nb[2];
+        num = num + czl * (fz ? 0.0 : k2) * (double)nc.nb[3];
+        den = 0.5 * mu + cxl * (fx ? kd : k0);
+        den = den + cyl * (fy ? kd : k0);
+        den = den + czl * (fz ? kd : k0);
+      }
+      if (divide) {
+        asm volatile("" : "+v"(num));  // a branch: the division is not worth computing beside the other
+        fnew = num / den;
+      }
+      const double fv = (double)(T)fnew;
+      h2 = h1;
+      h1 = fv;
+      // task k - 1's stores are older than this turn's five loads
+      wait_vm<5>();
+      publish(pub);
+      buf_store((T)fnew, __builtin_amdgcn_make_buffer_rsrc(fwin, 0, fbytes, kBufferWord3), voff_st, self_off(oc.w0));
+      if constexpr (kDC == 1)
+        buf_store((float)(fnew - fpv), __builtin_amdgcn_make_buffer_rsrc(rwin, 0, fbytes >> 1, kBufferWord3),
+                  voff_st == kOut ? kOut : voff_st >> 1, self_off(oc.w0) >> 1);
+      const double fz = voff_st == kOut ? 0.0 : fv;
+      buf_store(wave_sum4(fz, scx * fz, scy * fz, scz * fz), rp, voff_p, mom_off(oc.w1));
+      pub = base + (uint32_t)ox1(oc.w1);
+      if (want) polled(pv);
+      ++k;
+    };
+    // Nothing is in flight at the top: wait for task k's rows, load it and what
+    // may follow, and go on while tasks come loaded.  Every path to a task's
+    // update has issued the same loads after the task's own, so that a wait for
+    // those never covers younger ones.
+    while (k < n) {
+      wait_vm<0>();
+      publish(pub);
+      ro = rec_own(k);
+      rn = rec_nbr(k);
+      Own o0, o1, o2, o3;
+      Nbr n0, n1;
+      issue_own(o0, ro, k);
+      ro = rec_own(k + 1u);
+      n0.m = ld_mom(o0.w1);
+      {
+        const bool special = o0.w0 >> 31;
+        const bool fy = special && rn.x[1] & Geometry::kPenWaitY2, fz = special && rn.x[1] & Geometry::kPenWaitZ2;
+        const int32_t x = ox1(o0.w1);
+        const int32_t xy = o0.w1 & Geometry::kPenWaitY ? x : 0, xz = o0.w1 & Geometry::kPenWaitZ ? x : 0;
+        for (uint32_t it = 0; py < xy || pz < xz || fy || fz; ++it) {
+          polled(poll());
+          if (py >= xy && pz >= xz) {
+            if (!fy && !fz) break;
+            const uint32_t vy = pencil_poll(fy ? own - 2 * sy : own), vz = pencil_poll(fz ? own - 2 * sz : own);
+            if ((!fy || (int32_t)(__builtin_amdgcn_readfirstlane(vy) - base) >= x) &&
+                (!fz || (int32_t)(__builtin_amdgcn_readfirstlane(vz) - base) >= x))
+              break;
+          }
+          const uint32_t spin = args_now()->spin;
+          uint32_t* const err = st + 1;
+          if (it >= spin || ((it & 63u) == 63u && __builtin_amdgcn_readfirstlane(pencil_poll(err)) != 0u)) {
+            if (lane == 0 && it >= spin) {
+              err[1] = o;
+              err[2] = k;
+              err[3] = pen.id;
+              err[4] = u;
+              err[5] = base;
+              __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            alive = false;
+            break;
+          }
+          __builtin_amdgcn_s_sleep(kPenSleep);
+        }
+        if (!alive) break;
+      }
+      asm volatile("" ::: "memory");  // the loads stay after the polls that cleared them
+      issue_nb(n0, rn, o0.w0, o0.w1, fbytes);
+      rn = rec_nbr(k + 1u);
+      issue_own(o1, ro, k + 1u);
+      ro = rec_own(k + 2u);
+      issue_own(o2, ro, k + 2u);
+      ro = rec_own(k + 3u);
+      while (true) {
+        turn(o0, n0, o1, n1, o3);
+        if (n1.bytes == 0) break;
+        turn(o1, n1, o2, n0, o0);
+        if (n0.bytes == 0) break;
+        turn(o2, n0, o3, n1, o1);
+        if (n1.bytes == 0) break;
+        turn(o3, n1, o0, n0, o2);
+        if (n0.bytes == 0) break;
       }
     }
+    if (!alive) break;
+    done += n;
+    cl = claim();
+    // the row's last stores have reached L2: the whole row is done
+    wait_vm<0>();
+    publish(base + args_now()->Nx + 1u);
+    c = __builtin_amdgcn_readfirstlane(cl);
   }
-  }
-out:
-  if (lane == 0) {
-    a.diag[gridDim.x + blockIdx.x] = done;
-    __hip_atomic_fetch_add(a.done + o, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
+  if (lane == 0 && done) __hip_atomic_fetch_add(st + kPenOct * (1 + o) + kPenDone, done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ------------------------------------------------------------------ tiled sweep
@@ -1025,7 +1124,7 @@ template <typename T>
 struct TileArgs {
   T* f;                    // right-hand side 0
   const Mom* mom;
-  double* part;            // [cell][octant][4] partial moments; null = skip
+  double* part;            // [octant][cell][4] partial moments; null = skip
   const uint32_t* rec;     // this launch's first tile record
   const double* cx;
   const double* cy;
@@ -1093,10 +1192,10 @@ __global__ __launch_bounds__(64) void k_tile(TileArgs<T> a) {
   const uint32_t oob = len * cb;                            // the zero slot; stores there are dropped
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
       a.f + rhs * a.rs_f + (size_t)o * a.ostride + (size_t)lo * (uint32_t)Nc8, 0, (int)oob, kBufferWord3);
-  // partial moments of the tile's cells: [cell - cell_lo][octant][4] doubles
-  const uint32_t poob = cell_n * 256u;
+  // partial moments of the tile's cells: [cell - cell_lo][4] doubles of its octant
+  const uint32_t poob = cell_n * 32u;
   const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(
-      a.part ? a.part + (size_t)rhs * a.rs_mom * 32 + (size_t)cell_lo * 32 : nullptr, 0, a.part ? (int)poob : 0,
+      a.part ? a.part + ((size_t)rhs * 8 + o) * a.rs_mom * 4 + (size_t)cell_lo * 4 : nullptr, 0, a.part ? (int)poob : 0,
       kBufferWord3);
   const bool lact = lane < Nc8;
   const int ll = lact ? lane : 0;
@@ -1212,7 +1311,7 @@ __global__ __launch_bounds__(64) void k_tile(TileArgs<T> a) {
           }
         }
         buf_store(cc[s], rs, voff_st, sw ? lane_u32(r, tile_rec_slot(s)) * cb : oob);
-        buf_store(zz, rp, voff_p, sw ? ((cell - cell_lo) * 8u + o) * 32u : poob);
+        buf_store(zz, rp, voff_p, sw ? (cell - cell_lo) * 32u : poob);
       }
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
@@ -1240,7 +1339,7 @@ __global__ void k_commit(T* f, const T* fw, const int32_t* walls, int nwalls,
     const int32_t* wp = wall_pos + (size_t)w * Geometry::kWallPos;  // the wall cell per family
     const uint64_t vv = views[w];
     auto source = [&](int o, int src) -> const T* {
-      return src <= 8 ? f + (size_t)(src - 1) * d.ostride + (size_t)wp[ofam(src - 1)] * d.Nc8
+      return src <= 8 ? f + (size_t)(src - 1) * d.ostride + (size_t)wp[ofam(src - 1)] * d.vs
                       : fw + ((size_t)wall_corner[w] * 8 + o) * d.Nc8;
     };
     if (d.Nc8 <= kWave) {
@@ -1256,7 +1355,7 @@ __global__ void k_commit(T* f, const T* fw, const int32_t* walls, int nwalls,
 #pragma unroll
       for (int o = 0; o < 8; ++o) {
         const int src = (int)((vv >> (8 * o + 4)) & 15u);
-        if (src != 0 && lane < d.Nc8) f[(size_t)o * d.ostride + (size_t)wp[ofam(o)] * d.Nc8 + lane] = v[o];
+        if (src != 0 && lane < d.Nc8) f[(size_t)o * d.ostride + (size_t)wp[ofam(o)] * d.vs + lane] = v[o];
       }
       continue;
     }
@@ -1264,7 +1363,7 @@ __global__ void k_commit(T* f, const T* fw, const int32_t* walls, int nwalls,
       const int src = (int)((vv >> (8 * o + 4)) & 15u);
       if (src == 0) continue;
       const T* s = source(o, src);
-      T* dst = f + (size_t)o * d.ostride + (size_t)wp[ofam(o)] * d.Nc8;
+      T* dst = f + (size_t)o * d.ostride + (size_t)wp[ofam(o)] * d.vs;
       for (int l = lane; l < d.Nc8; l += kWave) dst[l] = s[l];
     }
   }
@@ -1396,8 +1495,8 @@ __device__ void wall_one(const WallArgs<T>& a, int idx, int lane) {
           n1 = load_nbr<T, COUPLED>(a, cell + st, oo, l, sidx[fa * 2]);
           n2 = load_nbr<T, COUPLED>(a, cell + 2 * st, oo, l, sidx[fa * 2 + 1]);
         } else {
-          n1 = (double)a.f[oo * os + (size_t)wp[4 + fa * 8 + q] * Nc8 + l];
-          n2 = (double)a.f[oo * os + (size_t)wp[4 + fa * 8 + 4 + q] * Nc8 + l];
+          n1 = (double)a.f[oo * os + (size_t)wp[4 + fa * 8 + q] * a.d.vs + l];
+          n2 = (double)a.f[oo * os + (size_t)wp[4 + fa * 8 + 4 + q] * a.d.vs + l];
         }
         const double val = e1 * n1 + e2 * n2;
         v[P.face[fa].store + oo] = val;
@@ -1415,7 +1514,7 @@ __device__ void wall_one(const WallArgs<T>& a, int idx, int lane) {
     for (int s = 0; s < 16; ++s) {
       if (!((written >> s) & 1u)) continue;
       if (s < 8)
-        a.f[s * os + (size_t)wp[ofam(s)] * Nc8 + l] = (T)v[s];
+        a.f[s * os + (size_t)wp[ofam(s)] * a.d.vs + l] = (T)v[s];
       else
         a.fw[((size_t)corner * 8 + (s - 8)) * Nc8 + l] = (T)v[s];
     }
@@ -1731,21 +1830,31 @@ __global__ __launch_bounds__(256) void k_planes(T* f, const double* w, double pd
 // ------------------------------------------------------------------ moments
 
 // Interior fluid cells: their f is final after the sweep, so the moments are
-// the sum of the eight octant partials.
+// the sum of the eight octant partials, each the sum of its `chunks` units of
+// 64 velocities.
 __global__ void k_moments_partials(const double* part, const int32_t* cells, int64_t n, Mom* mom,
-                                   int64_t ntotal) {
-  part += blockIdx.y * ntotal * 32;
+                                   int64_t ntotal, int chunks) {
+  part += blockIdx.y * ntotal * 32 * chunks;
   mom += blockIdx.y * ntotal;
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n;
        t += (int64_t)gridDim.x * blockDim.x) {
     const int64_t c = cells[t];
-    const double* p = part + (size_t)c * 32;
+    const double* p = part + (size_t)c * 4;
     double r = 0.0, x = 0.0, y = 0.0, z = 0.0;
     for (int q = 0; q < 8; ++q) {
-      r += p[q * 4 + 0];
-      x += p[q * 4 + 1];
-      y += p[q * 4 + 2];
-      z += p[q * 4 + 3];
+      const double* pq = p + (size_t)q * ntotal * 4;
+      double v0 = pq[0], v1 = pq[1], v2 = pq[2], v3 = pq[3];
+      for (int h = 1; h < chunks; ++h) {
+        const double* ph = pq + (size_t)h * ntotal * 32;
+        v0 += ph[0];
+        v1 += ph[1];
+        v2 += ph[2];
+        v3 += ph[3];
+      }
+      r += v0;
+      x += v1;
+      y += v2;
+      z += v3;
     }
     mom[c] = Mom{r, x, y, z};
   }
@@ -1914,7 +2023,7 @@ __global__ __launch_bounds__(256) void k_dc_slots(double* s, float* e, double* o
     const int64_t cnt = (int64_t)act_n[gw];
     for (int64_t j = 0; j < cnt; ++j) {
       const uint32_t w = act[gw + j * nw];
-      const size_t at = (size_t)(w >> 28) * d.ostride + (size_t)(w & 0x0fffffffu) * d.Nc8;
+      const size_t at = (size_t)(w >> 28) * d.ostride + (size_t)(w & 0x0fffffffu) * d.vs;
       for (int l = lane; l < d.Nc8; l += kWave) e[at + l] = flag ? r[at + l] : e[at + l] + r[at + l];
     }
     return;
@@ -1922,7 +2031,7 @@ __global__ __launch_bounds__(256) void k_dc_slots(double* s, float* e, double* o
   uint32_t rec = 0;  // slots this wave recorded (mode 1)
   for (int64_t idx = gw; idx < n; idx += nw) {
     const uint32_t w = list[idx];
-    const size_t at = (size_t)(w >> 28) * d.ostride + (size_t)(w & 0x0fffffffu) * d.Nc8;
+    const size_t at = (size_t)(w >> 28) * d.ostride + (size_t)(w & 0x0fffffffu) * d.vs;
     double* oo = old + (size_t)idx * d.Nc8;
     bool nz = false;
     for (int l = lane; l < d.Nc8; l += kWave) {
@@ -2091,6 +2200,33 @@ SweepKernel<T> sweep_kernel_dc(const Ctx& c, int rb) {
   }
 }
 
+// The pencil sweep's kernel for a defect-correction role (IterMode::dc).
+template <typename T>
+auto pencil_kernel(int dc) -> void (*)(PencilArgs<T>) {
+  if constexpr (sizeof(T) == sizeof(float)) return k_sweep_pencil<float, 2>;
+  else return dc ? k_sweep_pencil<double, 1> : k_sweep_pencil<double, 0>;
+}
+
+// Units of 64 velocities per octant.
+inline uint32_t pencil_chunks(const Dims& d) { return (uint32_t)((d.Nc8 + kWave - 1) / kWave); }
+
+// Progress words of a unit's octant: its rows, to a whole 128-byte line, so that
+// no line is written by two XCDs.
+inline size_t pencil_words(const Geometry& g) { return ((size_t)g.Ny * g.Nz + 31) / 32 * 32; }
+
+// Copies of the partial moments per right-hand side (one per unit of the
+// pencil sweep; the other sweeps add their velocity passes in place).
+inline int part_units(const Ctx& c) { return c.pencil ? (int)pencil_chunks(c.d) : 1; }
+
+// Units whose rows are taken together: one unit's rows keep about as many
+// waves busy as a strip's diagonal holds rows times the rows a wave-long
+// diagonal chain overlaps, so small images interleave several units.
+inline uint32_t pencil_group(const Ctx& c, uint32_t units) {
+  const int64_t rows = std::min<int64_t>(c.pen_rows, std::min(c.g.Ny, c.g.Nz));
+  const int64_t busy = std::max<int64_t>(1, rows * 16);
+  return (uint32_t)std::max<int64_t>(1, std::min<int64_t>(units, (c.pen_waves + busy - 1) / busy));
+}
+
 // Enqueue nsteps iterations on the context's stream.  With ev0 >= 0, four
 // events per step (steps ev0, ev0 + 1, ..., below kMaxTimedSteps) bracket the
 // sweep, boundary and moment phases; the caller synchronises and reads them.
@@ -2175,40 +2311,46 @@ int enqueue_t(Ctx& c, State<T>& st, int nsteps, int ev0, const IterMode& im) {
     // joined back into the context's stream: one chain's launches fill the
     // GPU while another's drain and start.  Without them the groups run one
     // after the other.
-    const bool flow = c.sweep_flow && sizeof(T) == sizeof(double) && im.dc == 0 && c.nrhs == 1;
-    if (flow) {
-      FlowArgs fa{};
-      fa.f = reinterpret_cast<double*>(st.f);
-      fa.mom = im.mom;
-      fa.part = sa.part;
-      fa.rec = c.flow_rec;
-      fa.flags = c.flow_flags;
-      fa.epoch = c.flow_epoch;
-      fa.err = c.flow_err;
-      fa.wave_ctr = c.flow_epoch + 8;
-      fa.done = c.flow_epoch + 16;
-      fa.mode = c.flow_epoch + 32;
-      fa.next = c.flow_epoch + 40;
-      fa.waves = (uint32_t)c.flow_waves;
-      fa.barrier = (uint32_t)c.flow_barrier;
-      fa.cx = c.dcx; fa.cy = c.dcy; fa.cz = c.dcz; fa.w = c.dw;
-      fa.coef = c.coef;
-      fa.fw = reinterpret_cast<const double*>(st.fw);
-      fa.mu0 = c.mu_r[0];
-      for (int q = 0; q < 9; ++q) fa.off[q] = c.flow_off[q];
-      fa.ostride = d.ostride;
-      fa.nslot = g.nstore + 1;
-      fa.spin = 1u << 20;  // about 1-2 s of polls 16 x 64 cycles apart, far beyond any wait of a sweep
-      fa.diag = c.flow_diag;
-      FlowCounts fc{};
-      for (int q = 0; q < 8; ++q) fc.n[q] = (uint32_t)(c.flow_off[q + 1] - c.flow_off[q]);
-      hipLaunchKernelGGL(k_flow_epoch, dim3(1), dim3(64), 0, c.stream, c.flow_epoch);
-      hipLaunchKernelGGL(c.flow_early ? k_sweep_flow<true> : k_sweep_flow<false>, dim3(8u * (unsigned)c.flow_waves),
-                         dim3(64), 0, c.stream, fa, fa.rec,
-                         fa.mom, fa.coef);
-      hipLaunchKernelGGL(k_flow_done, dim3(1), dim3(64), 0, c.stream, c.flow_epoch, fc);
+    if (c.pencil) {
+      const uint32_t chunks = pencil_chunks(d);
+      PencilArgs<T> pa{};
+      pa.f = st.f;
+      pa.fw = st.fw;
+      pa.part = sa.part;
+      pa.prog = c.pen_prog;
+      pa.st = c.pen_state;
+      pa.cx = c.dcx; pa.cy = c.dcy; pa.cz = c.dcz; pa.w = c.dw;
+      pa.mu = c.d_mu;
+      pa.ostride = d.ostride;
+      pa.rs_f = d.rs_f;
+      pa.rs_fw = d.rs_fw;
+      pa.rs_mom = d.Ntotal;
+      for (int q = 0; q < 9; ++q) pa.off[q] = (uint32_t)g.pen_off[q];
+      pa.vs = (uint32_t)d.vs;
+      pa.vs_fw = (uint32_t)d.Nc8;
+      pa.Nc8 = (uint32_t)d.Nc8;
+      pa.chunks = chunks;
+      pa.units = chunks * R;
+      pa.group = pencil_group(c, pa.units);
+      pa.Nx = (uint32_t)g.Nx;
+      pa.Ny = (uint32_t)g.Ny;
+      pa.c0 = sa.c0; pa.c1 = sa.c1; pa.c2 = sa.c2; pa.d1 = sa.d1;
+      pa.npen = (uint32_t)pencil_words(g);
+      pa.rec = c.pen_rec;
+      pa.pens = c.pen_list;
+      pa.mom = im.mom;
+      pa.spin = 1u << 20;  // seconds of polls, far beyond any wait of a sweep
+      pa.dc_r = c.r32.f;
+      pa.dc_e = c.s32.f;
+      pa.dc_fold = im.fold;
+      pa.dc_first = im.first;
+      PencilCounts pc{};
+      for (int q = 0; q < 8; ++q) pc.n[q] = (uint32_t)(g.pen_tasks[q] * pa.units);
+      hipLaunchKernelGGL(k_pencil_begin, dim3(1), dim3(64), 0, c.stream, c.pen_state, (uint32_t)g.Nx + 2u);
+      hipLaunchKernelGGL(pencil_kernel<T>(im.dc), dim3(8u * (unsigned)c.pen_waves), dim3(64), 0, c.stream, pa);
+      hipLaunchKernelGGL(k_pencil_done, dim3(1), dim3(64), 0, c.stream, c.pen_state, pc);
     }
-    const int ng = c.sweep_tiles || flow ? 0 : std::max(1, c.oct_groups);
+    const int ng = c.sweep_tiles || c.pencil ? 0 : std::max(1, c.oct_groups);
     const bool conc = ng > 1 && c.side[0] != nullptr;
     if (conc) {
       HIP_TRY(hipEventRecord(c.fork_ev, c.stream));
@@ -2310,7 +2452,7 @@ int enqueue_t(Ctx& c, State<T>& st, int nsteps, int ev0, const IterMode& im) {
       const int64_t ni = (int64_t)g.fluid_interior.size(), nbd = (int64_t)g.fluid_boundary.size();
       if (ni > 0)
         hipLaunchKernelGGL(k_moments_partials, dim3(grid_for(ni, 256), R), dim3(256), 0, c.stream,
-                           (const double*)c.part, c.fluid_int, ni, im.mom, g.Ntotal);
+                           (const double*)c.part, c.fluid_int, ni, im.mom, g.Ntotal, part_units(c));
       if (nbd > 0)
         hipLaunchKernelGGL(k_moments_direct<T>, dim3((unsigned)((nbd + wpb - 1) / wpb), R),
                            dim3(wpb * kWave), 0, c.stream, (const T*)st.f, c.fluid_bnd, nbd,
@@ -2454,7 +2596,7 @@ int iterate(Ctx& c, int nsteps) {
                : enqueue_t<double>(c, c.s64, nsteps, 0, IterMode{c.mom, c.prm.press_drop, 0, 0, 0});
   if (rc) return rc;
   HIP_TRY(hipStreamSynchronize(c.stream));
-  if ((rc = flow_check(c))) return rc;
+  if ((rc = pencil_check(c))) return rc;
   const int timed = std::min(nsteps, kMaxTimedSteps);
   if (timed > 0) {
     double acc[3] = {0, 0, 0};
@@ -2477,6 +2619,81 @@ int iterate(Ctx& c, int nsteps) {
 
 namespace piks {
 
+namespace {
+
+// Whether the context sweeps in one launch by rows (pencils): the default,
+// unless a setting that shapes the hyperplane or tiled sweep asks for those.
+// PIKS_SWEEP_FLOW=0 turns it off; =1 asks for it and is refused (ctx_create_device)
+// on anything but a single FP64 solve with 64 velocities per octant on a
+// context with its own stream.
+int sweep_choice(Ctx& c) {
+  const char* const shaping[] = {"PIKS_XCD_REMAP", "PIKS_SWEEP_BLOCK", "PIKS_SWEEP_TILES", "PIKS_SWEEP_GENERIC",
+                                 "PIKS_OCT_GROUPS", "PIKS_OCT_SERIAL", "PIKS_SWEEP_NT", "PIKS_SWEEP_RECIP"};
+  c.flow_req = c.prm.sweep != 0 ? 0 : -1;
+  for (const char* v : shaping)
+    if (std::getenv(v)) c.flow_req = 0;
+  if (const char* b = std::getenv("PIKS_SWEEP_FLOW")) c.flow_req = std::atoi(b) != 0 ? 1 : 0;
+  if (const char* b = std::getenv("PIKS_FLOW_WAVES")) {
+    const int v = std::atoi(b);
+    if (v < 8 || v > 4096) return fail(PIKS_E_ARG, "PIKS_FLOW_WAVES must be 8..4096");
+    c.pen_waves = v;
+  }
+  if (const char* b = std::getenv("PIKS_FLOW_STRIPS")) {
+    c.flow_strips = std::atoi(b);
+    if (c.flow_strips < 1 || c.flow_strips > 64) return fail(PIKS_E_ARG, "PIKS_FLOW_STRIPS must be 1..64");
+  }
+  c.pencil = c.flow_req != 0;
+  return 0;
+}
+
+// Rows of y per strip of the pencil sweep.
+int pencil_rows(const Ctx& c) {
+  if (c.flow_strips > 0) return std::max(1, (c.prm.ny + c.flow_strips - 1) / c.flow_strips);
+  return 1 << 20;
+}
+
+// Strides of f.  The pencil sweep's slots are whole 128-byte lines in every
+// precision the context holds, so that no line holds two slots (its kernel
+// reads finished slots through the L1 while others are being written).
+int slot_stride(const Ctx& c) {
+  const int nc8 = (int)c.cx.size(), line = c.prm.precision == PIKS_PREC_FP32_REFINED ? 32 : 16;
+  return c.pencil ? (nc8 + line - 1) / line * line : nc8;
+}
+
+void set_storage(Ctx& c) {
+  c.d.vs = slot_stride(c);
+  c.d.ostride = (c.g.nstore + 1) * (int64_t)c.d.vs;   // + the zero slot
+  c.n_f = (size_t)c.d.ostride * 8;
+  c.d.rs_f = (int64_t)c.n_f;
+}
+
+// The hyperplane sweep addresses one hyperplane's storage window with 32-bit
+// offsets: task records as it reads them, element offsets inside the
+// (hyperplane, octant) window, the zero slot as the window's end.
+int hyperplane_windows(Ctx& c) {
+  int64_t maxwin = 0;
+  for (int32_t v : c.g.hp_len) maxwin = std::max<int64_t>(maxwin, v);
+  if (maxwin * c.d.Nc8 * (int64_t)sizeof(double) >= ((int64_t)1 << 31))
+    return fail(PIKS_E_ARG, "a hyperplane's storage window exceeds 2 GiB (image or velocity grid too large)");
+  make_window_relative(c.g, c.d.Nc8, host_threads());
+  return 0;
+}
+
+// Give up the pencil sweep before anything is allocated: the hyperplane
+// schedule and its storage order.
+int use_hyperplanes(Ctx& c) {
+  Geometry& g = c.g;
+  c.pencil = false;
+  std::vector<Geometry::Pencil>().swap(g.pen);
+  std::vector<uint32_t>().swap(g.pen_rec);
+  build_sweep_schedule(g, host_threads());
+  set_storage(c);
+  if (c.prm.precision == PIKS_PREC_FP32_REFINED) c.ns_host = build_nonswept(g, host_threads());
+  return hyperplane_windows(c);
+}
+
+}  // namespace
+
 int ctx_create_host(const piks_params* p, const uint8_t* raw, int64_t nbytes, Ctx** out) {
   if (!p || !raw || !out) return fail(PIKS_E_ARG, "null argument");
   *out = nullptr;
@@ -2491,13 +2708,18 @@ int ctx_create_host(const piks_params* p, const uint8_t* raw, int64_t nbytes, Ct
   if (int rc = setup_velocity(*c)) return rc;
   std::string err;
   GeomInput gi{p->nx, p->ny, p->nz, p->fluid_layer, p->wall_ext_order};
+  if (int rc = sweep_choice(*c)) return rc;
+  if (c->pencil) {
+    gi.pencil_rows = c->pen_rows = pencil_rows(*c);
+    gi.pencil_vs = slot_stride(*c);
+  }
   if (p->wall_ext_order < 1 || p->wall_ext_order > 3)
     std::fprintf(stderr, " Error: wallExtOrder wroond shoud be [1|2|3]\n");  // src/physicalGrid.F90:947
   if (int rc = build_geometry(gi, raw, nbytes, c->g, err)) return fail(rc, err);
   const Geometry& g = c->g;
-  c->d = Dims{g.Nx, g.Ny, g.Nz, g.Nxt, g.Nxyt, g.Ntotal, (int)c->cx.size(), {}, 0};
-  c->d.ostride = (g.nstore + 1) * (int64_t)c->d.Nc8;   // + the zero slot
-  c->n_f = (size_t)c->d.ostride * 8;
+  c->pencil = g.raster;  // an image beyond the records' limits has the hyperplane schedule
+  c->d = Dims{g.Nx, g.Ny, g.Nz, g.Nxt, g.Nxyt, g.Ntotal, (int)c->cx.size(), 0, {}, 0};
+  set_storage(*c);
   c->n_fw = (size_t)std::max(g.ncorner, 1) * 8 * c->d.Nc8;
   c->n_buf = (size_t)g.Ny * g.Nz * 8 * c->d.Nc8;
   c->n_snap = std::max<size_t>(g.snap_cell.size(), 1) * 8 * c->d.Nc8;
@@ -2546,26 +2768,6 @@ int ctx_create_host(const piks_params* p, const uint8_t* raw, int64_t nbytes, Ct
   }
   if (const char* b = std::getenv("PIKS_OCT_SERIAL")) c->oct_serial = std::atoi(b) != 0;
   if (const char* b = std::getenv("PIKS_DC_ACTIVE")) c->dc_active = std::atoi(b) != 0;
-  // the single-launch sweep: on where it applies unless a setting that
-  // shapes the hyperplane sweep asks for that path; PIKS_SWEEP_FLOW=0 turns
-  // it off, =1 makes a context it cannot serve an error
-  const char* const shaping[] = {"PIKS_XCD_REMAP", "PIKS_SWEEP_BLOCK", "PIKS_SWEEP_TILES", "PIKS_SWEEP_GENERIC",
-                                 "PIKS_OCT_GROUPS", "PIKS_OCT_SERIAL", "PIKS_SWEEP_NT", "PIKS_SWEEP_RECIP"};
-  c->flow_req = p->sweep != 0 ? 0 : -1;
-  for (const char* v : shaping)
-    if (std::getenv(v)) c->flow_req = 0;
-  if (const char* b = std::getenv("PIKS_SWEEP_FLOW")) c->flow_req = std::atoi(b) != 0 ? 1 : 0;
-  if (const char* b = std::getenv("PIKS_FLOW_WAVES")) {
-    const int v = std::atoi(b);
-    if (v < 8 || v > 4096) return fail(PIKS_E_ARG, "PIKS_FLOW_WAVES must be 8..4096");
-    c->flow_waves = v;
-  }
-  if (const char* b = std::getenv("PIKS_FLOW_BARRIER")) c->flow_barrier = std::atoi(b);
-  if (const char* b = std::getenv("PIKS_FLOW_EARLY")) c->flow_early_req = std::atoi(b) != 0 ? 1 : 0;
-  if (const char* b = std::getenv("PIKS_FLOW_STRIPS")) {
-    c->flow_strips = std::atoi(b);
-    if (c->flow_strips < 1 || c->flow_strips > 64) return fail(PIKS_E_ARG, "PIKS_FLOW_STRIPS must be 1..64");
-  }
   if (const char* b = std::getenv("PIKS_MULTI_RB")) {
     const int v = std::atoi(b);
     if (v != 1 && v != 2 && v != 4) return fail(PIKS_E_ARG, "PIKS_MULTI_RB must be 1, 2 or 4");
@@ -2580,7 +2782,6 @@ int ctx_create_host(const piks_params* p, const uint8_t* raw, int64_t nbytes, Ct
   c->kn_r.assign(1, p->kn);
   c->mu_r.assign(1, c->mu);
   c->mass_r.assign(1, 1.0);
-  c->d.rs_f = (int64_t)c->n_f;
   c->d.rs_fw = (int64_t)c->n_fw;
   c->d.rs_buf = (int64_t)c->n_buf;
   c->d.rs_snap = (int64_t)c->n_snap;
@@ -2599,20 +2800,14 @@ int ctx_create_host(const piks_params* p, const uint8_t* raw, int64_t nbytes, Ct
     // every buffer offset of a tile (bytes, the zero slot included, and the
     // partial moments of its cells) is 32-bit
     if ((gt.tl_maxwin + 1) * c->d.Nc8 * (int64_t)sizeof(double) >= ((int64_t)1 << 31) ||
-        (gt.tl_maxspan + 1) * 256 >= ((int64_t)1 << 31)) {
+        (gt.tl_maxspan + 1) * 32 >= ((int64_t)1 << 31)) {
       c->sweep_tiles = false;
       gt.tl_rec.clear();
       gt.tl_rec.shrink_to_fit();
     }
   }
-  // the sweep addresses one hyperplane's storage window with 32-bit offsets
-  int64_t maxwin = 0;
-  for (int32_t v : g.hp_len) maxwin = std::max<int64_t>(maxwin, v);
-  if (maxwin * c->d.Nc8 * (int64_t)sizeof(double) >= ((int64_t)1 << 31))
-    return fail(PIKS_E_ARG, "a hyperplane's storage window exceeds 2 GiB (image or velocity grid too large)");
-  // task records as the sweep reads them: element offsets inside the
-  // (hyperplane, octant) window, the zero slot as the window's end
-  make_window_relative(c->g, c->d.Nc8, host_threads());
+  if (!c->pencil)
+    if (int rc = hyperplane_windows(*c)) return rc;
   *out = c.release();
   return 0;
 }
@@ -2629,156 +2824,81 @@ size_t ctx_device_bytes(const Ctx& c) {
                                        R * (size_t)g.Ntotal * 3 * sizeof(Mom) + (size_t)c.n_ns * 4 +
                                        R * ((size_t)c.n_ns + 262144) * 4
                                  : 0;
-  const size_t per_cell = (size_t)g.Ntotal * (R * (sizeof(Mom) + 32 * sizeof(double)) + 1 + 4 + 4 * 4);
+  const size_t per_cell = (size_t)g.Ntotal * (R * (sizeof(Mom) + 32 * sizeof(double) * part_units(c)) + 1 + 4 + 4 * (c.pencil ? 1 : 4));
   const size_t walls = g.wall_cell.size() * (8 + 4 + 4 + 1 + 8 + 8) + g.wall_pos.size() * 4 +
                        g.uncoupled.size() * 4 +
                        g.coupled.size() * 4 * 7 + g.snap_cell.size() * 4 + g.commit_walls.size() * 4;
   const size_t fluid = (size_t)(g.fluid_interior.size() + g.fluid_boundary.size()) * 8 + g.surface.size() * 4;
-  const size_t sched = c.sweep_tiles ? g.tl_rec.size() * 4 : g.hp_task.size() * 4 + g.hp_lo.size() * 16;
+  const size_t sched = c.pencil ? g.pen_rec.size() * 4 + g.pen.size() * sizeof(Geometry::Pencil) +
+                                      R * pencil_chunks(c.d) * 8 * pencil_words(g) * 4
+                       : c.sweep_tiles ? g.tl_rec.size() * 4 : g.hp_task.size() * 4 + g.hp_lo.size() * 16;
   return state64 + state32 + per_cell + walls + fluid + sched +
          R * ((size_t)g.Ny * g.Nz * 8 + 8) + 4 * c.cx.size() * 8 + 64 * 256;
 }
 
-// The single-launch sweep's schedule and state, refused unless the context
-// can use it: FP64 single solve, 64 velocities per octant, its own stream,
-// slot indices below 2^28, W waves per octant resident at once (probe
-// launches of the kernel itself) and W blocks on each of the eight XCDs (a
-// probe launch of the same grid reads each block's XCD id).  Records:
-// octant o's tasks in hyperplane order; words 1..6 the upwind sources
-// (flow_source): the neighbours' slot indices, with bit 31 set on the
-// nearest swept neighbour along each axis (the one the task waits for), and
-// reads of wall slots the reference switched resolved to their source.
-int64_t tasks_per_hyperplane(const Geometry& g);
-
-int flow_setup(Ctx& c) {
-  const Geometry& g = c.g;
-  const int64_t nc8 = c.d.Nc8, ns = g.nstore;
-  if (c.nrhs != 1 || nc8 != 64 || c.stream_ordered || c.prm.precision != PIKS_PREC_FP64 || ns + 1 >= (1 << 28))
-    return fail(PIKS_E_ARG, "PIKS_SWEEP_FLOW needs a single FP64 solve with 64 velocities per octant on a "
-                            "context with its own stream");
-  // waves per octant: all resident at once (one-wave workgroups).  The
-  // occupancy query is only an upper bound (it allowed 7 waves per SIMD where
-  // 6 were resident), so a probe launch of the sweep kernel itself, with the
-  // same registers, checks that every block of the grid is resident at once,
-  // and fewer waves are tried if not.
-  // Two loop structures (k_sweep_flow<kEarly>), each with its own registers:
-  // the early upwind loads pay where an octant's hyperplanes average at least
-  // two tasks per wave (measured: 40^3 and 64^3 packs faster without, 100^3
-  // and 200^3 with), so the choice follows W, and the probe is repeated for
-  // the kernel that will run.
-  using FlowKernel = void (*)(FlowArgs, const TaskRec*, const Mom*, const SweepCoef*);
+// Whether the pencil sweep can run on the context's device: the sweep needs
+// blocks on each of eight XCDs (blocks are dealt to them in turn), numbered
+// as the hardware id reads.  Sizes its launch: the waves per octant (XCD) that
+// fit the device at once, at most one per row and unit.
+int pencil_probe(Ctx& c, bool* usable) {
+  *usable = false;
   int per_cu = 0, dev = 0;
-  HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_sweep_flow<false>, 64, 0));
+  const bool refined = c.prm.precision == PIKS_PREC_FP32_REFINED;
+  if (refined)
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (k_sweep_pencil<float, 2>), 64, 0));
+  else
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (k_sweep_pencil<double, 0>), 64, 0));
   hipDeviceProp_t prop;
   HIP_TRY(hipGetDevice(&dev));
   HIP_TRY(hipGetDeviceProperties(&prop, dev));
-  const int64_t resident = (int64_t)per_cu * prop.multiProcessorCount;
-  const bool forced = c.flow_waves != 0;
-  if (!forced) c.flow_waves = (int)std::min<int64_t>(resident / 8, 1024);
-  if (c.flow_waves < 1 || 8 * (int64_t)c.flow_waves > resident)
-    return fail(PIKS_E_ARG, "PIKS_SWEEP_FLOW: " + std::to_string(c.flow_waves) + " waves per octant do not fit the " +
-                                std::to_string(resident) + " resident waves");
-  int rc = 0;
-  if ((rc = dalloc(c, &c.flow_epoch, 64)) || (rc = dalloc(c, &c.flow_diag, 2 * 8 * (size_t)c.flow_waves)))
-    return rc;
-  // flow_epoch: the launch's state (k_flow_epoch)
-  c.flow_err = c.flow_epoch + 1;
-  auto probe_waves = [&](FlowKernel kern) -> int {
-    for (int attempt = 0;; ++attempt) {
-      const unsigned nbp = 8u * (unsigned)c.flow_waves;
-      FlowArgs pa{};
-      pa.done = c.flow_epoch + 16;
-      pa.diag = c.flow_diag;
-      pa.probe = 1u << 12;  // about 1.4 ms; a launch places its blocks within tens of microseconds
-      std::vector<uint32_t> seen(nbp, 0);
-      HIP_TRY(hipMemsetAsync(c.flow_epoch, 0, 64 * sizeof(uint32_t), c.stream));
-      hipLaunchKernelGGL(kern, dim3(nbp), dim3(64), 0, c.stream, pa, nullptr, nullptr, nullptr);
-      HIP_TRY(hipMemcpyAsync(seen.data(), c.flow_diag, nbp * sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream));
-      HIP_TRY(hipStreamSynchronize(c.stream));
-      // a block that gave up saw the arrivals up to then; the first to give
-      // up saw only blocks that were resident together (none had left yet),
-      // so the smallest count is what fits at once
-      uint32_t fit = 0xffffffffu;
-      for (uint32_t v : seen) fit = std::min(fit, v);
-      if (fit == 0xffffffffu) return 0;
-      const int w = (int)(fit / 8) - 8 * attempt;
-      if (forced || attempt == 3 || w < 8)
-        return fail(PIKS_E_HIP, "single-launch sweep: " + std::to_string(nbp) + " one-wave blocks are not "
-                                "resident at once (" + std::to_string(fit) + " were)");
-      c.flow_waves = std::min(w, c.flow_waves - 8);
-    }
-  };
-  if ((rc = probe_waves(k_sweep_flow<false>))) return rc;
-  if (c.flow_early_req >= 0) c.flow_early = c.flow_early_req != 0;
-  else c.flow_early = tasks_per_hyperplane(g) / 8 >= 2 * (int64_t)c.flow_waves;
-  if (c.flow_early && (rc = probe_waves(k_sweep_flow<true>))) return rc;
-  const unsigned nb = 8u * (unsigned)c.flow_waves;
-  {
-    uint32_t* probe = nullptr;
-    HIP_TRY(hipMalloc(&probe, nb * sizeof(uint32_t)));
-    std::vector<uint32_t> xcc(nb, 99u);
-    hipLaunchKernelGGL(k_flow_probe, dim3(nb), dim3(64), 0, c.stream, probe, nb);
-    hipError_t e = hipMemcpyAsync(xcc.data(), probe, nb * sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
-    (void)hipFree(probe);
-    if (e != hipSuccess) return fail(PIKS_E_HIP, std::string("flow probe: ") + hipGetErrorString(e));
-    // the sweep needs W waves on every XCD (blocks are dealt to the XCDs in
-    // turn, from a start that varies between launches)
-    std::vector<unsigned> per(16, 0);
-    for (unsigned b = 0; b < nb; ++b) ++per[xcc[b] & 15u];
-    for (unsigned x = 0; x < 8; ++x)
-      if (per[x] != (unsigned)c.flow_waves)
-        return fail(PIKS_E_HIP, "single-launch sweep: XCD " + std::to_string(x) + " ran " + std::to_string(per[x]) +
-                                    " of the probe's " + std::to_string(nb) + " blocks, not " +
-                                    std::to_string(c.flow_waves));
+  if (c.pen_waves == 0) {
+    int64_t rows = 1;
+    for (int o = 0; o < 8; ++o) rows = std::max<int64_t>(rows, c.g.pen_off[o + 1] - c.g.pen_off[o]);
+    // Twelve waves per CU: fewer leave memory latency uncovered, more spread the
+    // rows in flight beyond what the L2 holds and make each trail its neighbours
+    // longer.  200^3 pack sweep at 8, 10, 12, 20 waves per CU: 12.6, 11.7, 11.5,
+    // 13.3 ms; 64^3: 0.88, 0.86, 0.87, 1.00 ms (shared counter lines still).
+    const int64_t fit = std::max<int64_t>(8, (int64_t)std::min(per_cu, 12) * prop.multiProcessorCount / 8);
+    c.pen_waves = (int)std::max<int64_t>(8, std::min<int64_t>(fit, rows * c.nrhs * pencil_chunks(c.d)));
   }
-  std::vector<int32_t> rec;
-  std::string err;
-  if ((rc = build_flow_records(g, (int)nc8, rec, c.flow_off, err, c.flow_strips))) return fail(rc, err);
-  static_assert(sizeof(TaskRec) == Geometry::kTaskWords * sizeof(int32_t), "one record per task");
-  if ((rc = dalloc(c, &c.flow_rec, rec.size() / Geometry::kTaskWords))) return rc;
-  HIP_TRY(hipMemcpyAsync(c.flow_rec, rec.data(), rec.size() * sizeof(int32_t), hipMemcpyHostToDevice, c.stream));
-  if ((rc = dalloc(c, &c.flow_flags, (size_t)8 * (ns + 1)))) return rc;
-  HIP_TRY(hipMemsetAsync(c.flow_flags, 0, (size_t)8 * (ns + 1) * sizeof(uint32_t), c.stream));
-  HIP_TRY(hipMemsetAsync(c.flow_epoch, 0, 64 * sizeof(uint32_t), c.stream));
-  HIP_TRY(hipStreamSynchronize(c.stream));  // the host vectors above end here
+  const unsigned nb = 8u * 64u;
+  std::vector<uint32_t> xcc(nb, 99u);
+  uint32_t* probe = nullptr;
+  HIP_TRY(c.stream_ordered ? hipMallocAsync((void**)&probe, nb * sizeof(uint32_t), c.stream)
+                           : hipMalloc((void**)&probe, nb * sizeof(uint32_t)));
+  hipLaunchKernelGGL(k_xcd_probe, dim3(nb), dim3(64), 0, c.stream, probe, nb);
+  hipError_t e = hipMemcpyAsync(xcc.data(), probe, nb * sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+  if (c.stream_ordered) (void)hipFreeAsync(probe, c.stream);
+  else (void)hipFree(probe);
+  if (e != hipSuccess) return fail(PIKS_E_HIP, std::string("XCD probe: ") + hipGetErrorString(e));
+  std::vector<unsigned> per(16, 0);
+  for (unsigned b = 0; b < nb; ++b) ++per[xcc[b] & 15u];
+  *usable = true;
+  for (unsigned x = 0; x < 8; ++x)
+    if (per[x] == 0) *usable = false;
   return 0;
 }
 
-// A failed wait of the single-launch sweep (its err flag), after the
-// context's stream has been synchronised: the iteration's result is not
-// valid; the context goes back to hyperplane launches.
-int flow_check(Ctx& c) {
-  if (!c.sweep_flow) return 0;
-  uint32_t err[6] = {0, 0, 0, 0, 0, 0};
-  HIP_TRY(hipMemcpy(err, c.flow_err, sizeof(err), hipMemcpyDeviceToHost));
-  if (!err[0]) return 0;
-  c.sweep_flow = false;
-  const size_t nb = 8 * (size_t)c.flow_waves;
-  std::vector<uint32_t> dg(2 * nb);
-  HIP_TRY(hipMemcpy(dg.data(), c.flow_diag, dg.size() * 4, hipMemcpyDeviceToHost));
-  // diag: block b swept octant dg[b] and did dg[nb + b] tasks
-  std::vector<uint64_t> per(8, 0), done(8, 0);
-  for (size_t b = 0; b < nb; ++b) {
-    ++per[dg[b] & 7u];
-    done[dg[b] & 7u] += dg[nb + b];
-  }
-  std::string blocks, tasks;
-  for (int o = 0; o < 8; ++o) {
-    blocks += " " + std::to_string(per[(size_t)o]);
-    tasks += " " + std::to_string(done[(size_t)o]) + "/" + std::to_string(c.flow_off[o + 1] - c.flow_off[o]);
-  }
+// The message of a pencil sweep's failure state (words st[1..6]).
+int pencil_failure(const uint32_t* err) {
   const std::string what =
-      err[3] == 0xffffffffu   ? "octant " + std::to_string(err[1]) + " did " + std::to_string(err[2]) + " of its " +
-                                  std::to_string(err[4]) + " tasks"
-      : err[3] == 0xfffffffeu ? "XCD " + std::to_string(err[1]) + " started wave " + std::to_string(err[2]) +
-                                    " of " + std::to_string(err[4])
-                              : "a dependency wait gave up (octant " + std::to_string(err[1]) + ", task " + std::to_string(err[2]) +
-                ", slot " + std::to_string(err[3]) + ", epoch " + std::to_string(err[4]) + ", flag seen " +
-                std::to_string(err[5]) + ")";
-  return fail(PIKS_E_HIP, "single-launch sweep: " + what + "; blocks per octant" + blocks + "; tasks done" + tasks +
-                              "; the iteration's result is not valid and the context uses hyperplane launches "
-                              "from now on");
+      err[4] == 0xffffffffu
+          ? "octant " + std::to_string(err[1]) + " did " + std::to_string(err[2]) + " of its " + std::to_string(err[3]) +
+                " tasks"
+          : "a dependency wait gave up (octant " + std::to_string(err[1]) + ", task " + std::to_string(err[2]) +
+                " of row " + std::to_string(err[3]) + ", unit " + std::to_string(err[4]) + ")";
+  return fail(PIKS_E_HIP, "single-launch sweep: " + what + "; the state is not valid any more");
+}
+
+// A failed wait of the pencil sweep, after the context's stream has been
+// synchronised: the iteration's result, and so the context's state, is not
+// valid.
+int pencil_check(Ctx& c) {
+  if (!c.pencil) return 0;
+  uint32_t err[6] = {0, 0, 0, 0, 0, 0};
+  HIP_TRY(hipMemcpy(err, c.pen_state + 1, sizeof(err), hipMemcpyDeviceToHost));
+  return err[0] ? pencil_failure(err) : 0;
 }
 
 // Average sweep tasks (swept cell, octant) per oriented hyperplane.
@@ -2795,6 +2915,21 @@ int ctx_create_device(Ctx& c, hipStream_t stream) {
   } else {
     HIP_TRY(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
     c.own_stream = true;
+  }
+  if (c.flow_req == 1 &&
+      (c.nrhs != 1 || c.d.Nc8 != kWave || c.stream_ordered || c.prm.precision != PIKS_PREC_FP64))
+    return fail(PIKS_E_ARG, "PIKS_SWEEP_FLOW needs a single FP64 solve with 64 velocities per octant on a "
+                            "context with its own stream");
+  if (c.pencil) {
+    bool usable = false;
+    if (int rc = pencil_probe(c, &usable)) return rc;
+    if (c.nrhs > 1 && c.multi_rb > 0) usable = false;  // a layout of the hyperplane sweep is asked for
+    if (!usable) {
+      if (c.flow_req == 1) return fail(PIKS_E_HIP, "single-launch sweep: the device does not deal blocks to eight XCDs");
+      if (int rc = use_hyperplanes(c)) return rc;
+    }
+  }
+  if (c.own_stream) {
     size_t free_b = 0, total_b = 0;
     HIP_TRY(hipMemGetInfo(&free_b, &total_b));
     const size_t need = ctx_device_bytes(c);
@@ -2814,7 +2949,7 @@ int ctx_create_device(Ctx& c, hipStream_t stream) {
   // coming from the slots.
   if (c.oct_groups == 0) {
     const int64_t per_hp = tasks_per_hyperplane(c.g) * c.nrhs;
-    c.oct_groups = !stream && per_hp >= 10000 ? 4 : 1;
+    c.oct_groups = !c.pencil && !stream && per_hp >= 10000 ? 4 : 1;
   }
   if (c.oct_groups > 1 && !c.oct_serial) {
     // default priority, like the context's stream
@@ -2849,7 +2984,7 @@ int ctx_create_device(Ctx& c, hipStream_t stream) {
     c.phase = PIKS_PREC_FP32_REFINED;
   }
   if ((rc = dalloc(c, &c.mom, R * (size_t)g.Ntotal))) return rc;
-  if ((rc = dalloc(c, &c.part, R * (size_t)g.Ntotal * 32))) return rc;
+  if ((rc = dalloc(c, &c.part, R * (size_t)g.Ntotal * 32 * part_units(c)))) return rc;
   if ((rc = dalloc(c, &c.plane, R * (size_t)g.Ny * g.Nz))) return rc;
   if ((rc = upload(c, &c.d_mu, c.mu_r))) return rc;
   {
@@ -2891,7 +3026,16 @@ int ctx_create_device(Ctx& c, hipStream_t stream) {
   std::vector<int32_t> all(g.fluid_interior);
   all.insert(all.end(), g.fluid_boundary.begin(), g.fluid_boundary.end());
   if ((rc = upload(c, &c.fluid_all, all))) return rc;
-  if (c.sweep_tiles) {
+  if (c.pencil) {
+    static_assert(sizeof(TaskRec) == Geometry::kTaskWords * sizeof(uint32_t), "one record per task");
+    const size_t nrec = g.pen_rec.size() / Geometry::kTaskWords;
+    if ((rc = dalloc(c, &c.pen_rec, nrec + kPenPad))) return rc;
+    if (nrec)
+      HIP_TRY(hipMemcpyAsync(c.pen_rec, g.pen_rec.data(), nrec * sizeof(TaskRec), hipMemcpyHostToDevice, c.stream));
+    if ((rc = upload(c, &c.pen_list, g.pen)) || (rc = dalloc(c, &c.pen_state, kPenState)) ||
+        (rc = dalloc(c, &c.pen_prog, R * pencil_chunks(c.d) * 8 * pencil_words(g))))
+      return rc;
+  } else if (c.sweep_tiles) {
     if ((rc = upload(c, &c.tl_rec, g.tl_rec))) return rc;
   } else {
     if ((rc = upload(c, &c.hp_task, g.hp_task))) return rc;
@@ -2903,16 +3047,11 @@ int ctx_create_device(Ctx& c, hipStream_t stream) {
       win[q].pad = 0;
     }
     if ((rc = upload(c, &c.hp_win, win))) return rc;
-    if (c.flow_req != 0) {
-      const int r = flow_setup(c);
-      if (r == 0) c.sweep_flow = true;
-      else if (c.flow_req == 1) return r;
-      else set_error(0, "");  // automatic choice: the hyperplane launches serve, and no error stays behind
-    }
   }
   for (int F = 0; F < 4; ++F) {
-    if ((rc = upload(c, &c.pos[F], g.pos[F]))) return rc;
-    c.d.pos[F] = c.pos[F];
+    if (F == 0 || !g.raster)
+      if ((rc = upload(c, &c.pos[F], g.pos[F]))) return rc;
+    c.d.pos[F] = c.pos[g.raster ? 0 : F];
   }
   {
     std::vector<ViewArgs<double>> v64(1, ViewArgs<double>{c.s64.f, c.s64.fw, c.lab, c.wid, c.views, c.wall_corner, c.d});
@@ -2998,6 +3137,16 @@ int ctx_enqueue_plane(Ctx& c, double* host_plane) {
   HIP_TRY(hipMemcpyAsync(host_plane, c.plane, (size_t)g.Ny * g.Nz * c.nrhs * sizeof(double),
                          hipMemcpyDeviceToHost, c.stream));
   return 0;
+}
+
+int ctx_enqueue_state(Ctx& c, uint32_t* host_words) {
+  if (!c.pencil) return 0;
+  HIP_TRY(hipMemcpyAsync(host_words, c.pen_state + 1, kPenErrWords * sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream));
+  return 0;
+}
+
+int ctx_state_check(const Ctx& c, const uint32_t* host_words) {
+  return c.pencil && host_words[0] ? pencil_failure(host_words) : 0;
 }
 
 double ctx_mass(const Ctx& c, const double* u) {
@@ -3103,7 +3252,7 @@ int piks_iterate(void* ctx, int32_t nsteps) {
   if (c.use_graph) {
     if (int rc = ctx_enqueue(c, nsteps)) return rc;
     HIP_TRY(hipStreamSynchronize(c.stream));
-    return flow_check(c);
+    return pencil_check(c);
   }
   return iterate(c, nsteps);
 }
@@ -3268,9 +3417,9 @@ int piks_get_f(void* ctx, double* f) {
   HIP_TRY(hipStreamSynchronize(c.stream));
   // device [o][storage index][l] -> Fortran f(cell, l, o)
   for (size_t o = 0; o < 8; ++o) {
-    const std::vector<int32_t>& pos = c.g.pos[ofam((int)o)];
+    const std::vector<int32_t>& pos = c.g.opos((int)o);
     for (size_t cell = 0; cell < nt; ++cell) {
-      const double* src = &h[o * (size_t)c.d.ostride + (size_t)pos[cell] * nc8];
+      const double* src = &h[o * (size_t)c.d.ostride + (size_t)pos[cell] * (size_t)c.d.vs];
       for (size_t l = 0; l < nc8; ++l) f[(o * nc8 + l) * nt + cell] = src[l];
     }
   }
@@ -3320,7 +3469,8 @@ int piks_get_info(void* ctx, piks_info* info) {
   info->precision = c.phase;
   info->steps_fp32 = c.dc_inner;
   info->dc_block = c.phase == PIKS_PREC_FP32_REFINED ? c.dc_len : 0;
-  info->sweep_path = c.sweep_flow ? 2 : c.sweep_tiles ? 1 : 0;
+  info->sweep_path = c.pencil && c.nrhs == 1 && c.d.Nc8 == kWave && c.prm.precision == PIKS_PREC_FP64 ? 2
+                     : c.sweep_tiles ? 1 : 0;
   return 0;
 }
 

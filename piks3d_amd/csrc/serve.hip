@@ -65,10 +65,14 @@ struct Request {
   Clock::time_point t_submit, t_admit, t_done;
 };
 
+// room of the failure state's words in front of a slot's plane
+constexpr size_t kStateDoubles = 8;
+static_assert(kStateDoubles * sizeof(double) >= kPenErrWords * sizeof(uint32_t), "failure state");
+
 struct Slot {
   hipStream_t stream = nullptr;
   hipEvent_t done = nullptr;
-  double* plane = nullptr;  // pinned
+  double* plane = nullptr;  // pinned: kStateDoubles of the sweep's failure state, then the plane
   size_t plane_cap = 0;
   Request* req = nullptr;
 };
@@ -145,7 +149,8 @@ int enqueue_chunk(Slot& sl, Request& r) {
   const int chk = c.prm.chk_converge_step;
   r.chunk = std::min(chk - r.step % chk, r.max_step - r.step);
   if (int rc = ctx_enqueue(c, r.chunk)) return rc;
-  if (int rc = ctx_enqueue_plane(c, sl.plane)) return rc;
+  if (int rc = ctx_enqueue_plane(c, sl.plane + kStateDoubles)) return rc;
+  if (int rc = ctx_enqueue_state(c, reinterpret_cast<uint32_t*>(sl.plane))) return rc;
   if (hipEventRecord(sl.done, sl.stream) != hipSuccess) return set_error(PIKS_E_HIP, "hipEventRecord failed");
   return 0;
 }
@@ -173,13 +178,14 @@ void fail_request(Server& s, Slot& sl, Request& r, int rc) {
 // without the lock).
 void on_chunk_done(Server& s, Slot& sl, Request& r) {
   Ctx& c = *r.ctx;
+  if (int rc = ctx_state_check(c, reinterpret_cast<const uint32_t*>(sl.plane))) return fail_request(s, sl, r, rc);
   const int step = r.step + r.chunk;
   const int chk = c.prm.chk_converge_step;
   bool done = false, converged = false;
   double mass = r.mass, perm = r.perm, error = r.error;
   if (step % chk == 0) {
     double out[3];
-    ctx_check(c, 0, ctx_mass(c, sl.plane), out);
+    ctx_check(c, 0, ctx_mass(c, sl.plane + kStateDoubles), out);
     ctx_dc_policy(c, out[2]);  // FP32_REFINED: the next defect-correction blocks
     mass = out[0];
     perm = out[1];
@@ -215,7 +221,7 @@ void on_chunk_done(Server& s, Slot& sl, Request& r) {
 
 // Device set-up of an admitted request on its slot (called without the lock).
 void start_request(Server& s, Slot& sl, Request& r) {
-  const size_t need = (size_t)r.ctx->g.Ny * r.ctx->g.Nz;
+  const size_t need = kStateDoubles + (size_t)r.ctx->g.Ny * r.ctx->g.Nz;
   if (need > sl.plane_cap) {
     if (sl.plane) (void)hipHostFree(sl.plane);
     sl.plane = nullptr;
