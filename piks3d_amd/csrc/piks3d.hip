@@ -670,7 +670,7 @@ struct PencilArgs {
   const T* fw;              // corner store [corner][octant][velocity]
   double* part;             // [unit][octant][cell][4] partial moments; null = skip
   uint32_t* prog;           // [unit][octant][row]: progress
-  uint32_t* st;             // the launch's state (k_pencil_begin)
+  uint32_t* st;             // the launch's state (k_pencil_done prepares the next)
   const double* cx;
   const double* cy;
   const double* cz;
@@ -702,29 +702,27 @@ constexpr size_t kPenPad = 4;
 constexpr int kPenDone = 1, kPenNext = 0, kPenOct = 32, kPenState = 9 * kPenOct;
 static_assert(kPenErrWords == 6, "st[1..6]");
 
-// Next progress base; the counters of the launch cleared.
-__global__ void k_pencil_begin(uint32_t* st, uint32_t step) {
-  if (threadIdx.x == 0) __hip_atomic_fetch_add(st, step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if (threadIdx.x < 8) {
-    uint32_t* const q = st + kPenOct * (1 + threadIdx.x);
-    q[kPenNext] = q[kPenDone] = 0u;
-  }
-}
-
-// After the sweep: every octant's tasks done (else err, unless already set).
+// After the sweep: every octant's tasks done (else err, unless already set);
+// then the next launch's progress base, beyond this one's words, and counters
+// (a context starts with words, base and counters 0: no row done).  One launch
+// for both, where a second one before the sweep took 4 us of each iteration.
 struct PencilCounts {
   uint32_t n[8];
 };
-__global__ void k_pencil_done(uint32_t* st, PencilCounts c) {
+__global__ void k_pencil_done(uint32_t* st, PencilCounts c, uint32_t step) {
   const uint32_t o = threadIdx.x;
-  const uint32_t done = o < 8 ? st[kPenOct * (1 + o) + kPenDone] : 0u;
-  if (o < 8 && done != c.n[o] &&
-      __hip_atomic_fetch_add(st + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) {
-    st[2] = o;
-    st[3] = done;
-    st[4] = c.n[o];
-    st[5] = 0xffffffffu;
+  if (o < 8) {
+    uint32_t* const q = st + kPenOct * (1 + o);
+    const uint32_t done = q[kPenDone];
+    if (done != c.n[o] && __hip_atomic_fetch_add(st + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u) {
+      st[2] = o;
+      st[3] = done;
+      st[4] = c.n[o];
+      st[5] = 0xffffffffu;
+    }
+    q[kPenNext] = q[kPenDone] = 0u;
   }
+  if (o == 0) __hip_atomic_fetch_add(st, step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // XCD of every block of a grid of n one-wave blocks.
@@ -2350,9 +2348,8 @@ int enqueue_t(Ctx& c, State<T>& st, int nsteps, int ev0, const IterMode& im) {
       pa.dc_first = im.first;
       PencilCounts pc{};
       for (int q = 0; q < 8; ++q) pc.n[q] = (uint32_t)(g.pen_tasks[q] * pa.units);
-      hipLaunchKernelGGL(k_pencil_begin, dim3(1), dim3(64), 0, c.stream, c.pen_state, (uint32_t)g.Nx + 2u);
       hipLaunchKernelGGL(pencil_kernel<T>(im.dc), dim3(8u * (unsigned)c.pen_waves), dim3(64), 0, c.stream, pa);
-      hipLaunchKernelGGL(k_pencil_done, dim3(1), dim3(64), 0, c.stream, c.pen_state, pc);
+      hipLaunchKernelGGL(k_pencil_done, dim3(1), dim3(64), 0, c.stream, c.pen_state, pc, (uint32_t)g.Nx + 2u);
     }
     const int ng = c.sweep_tiles || c.pencil ? 0 : std::max(1, c.oct_groups);
     const bool conc = ng > 1 && c.side[0] != nullptr;
