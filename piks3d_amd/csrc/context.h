@@ -125,7 +125,7 @@ struct Ctx {
   TaskRec* pen_rec = nullptr;         // Geometry::pen_rec
   Geometry::Pencil* pen_list = nullptr;  // Geometry::pen
   uint32_t* pen_prog = nullptr;       // [unit][octant][row]: progress
-  uint32_t* pen_state = nullptr;      // the launch's state (k_pencil_done)
+  uint32_t* pen_state = nullptr;      // the launch's state (pencil_done)
   int multi_rb = 0;            // right-hand sides per wave of the several-Kn sweep (0: 1,
                                // measured fastest: 1, 2, 4 took 14.1, 14.8, 16.1 s on 16 Kn)
   int oct_groups = 0;          // octant groups of the sweep (1, 2, 4, 8; 0: 4 on a context

@@ -638,7 +638,7 @@ __global__ __launch_bounds__(64) void k_sweep1_rhs(SweepArgs<T> a) { sweep1_task
 // value is followed by its store, which updates that CU's L1; slots are whole
 // cache lines, see Dims::vs), and the L1 starts the launch invalidated.
 // Every wait gives up after `spin` polls (a safety net: it sets err and the
-// wave ends, so the grid always drains); k_pencil_done then checks that every
+// wave ends, so the grid always drains); k_halo (pencil_done) then checks that every
 // octant's tasks were done.
 //
 // The update is sweep1_task's, operation for operation.  Where no axis is
@@ -670,7 +670,7 @@ struct PencilArgs {
   const T* fw;              // corner store [corner][octant][velocity]
   double* part;             // [unit][octant][cell][4] partial moments; null = skip
   uint32_t* prog;           // [unit][octant][row]: progress
-  uint32_t* st;             // the launch's state (k_pencil_done prepares the next)
+  uint32_t* st;             // the launch's state (pencil_done prepares the next)
   const double* cx;
   const double* cy;
   const double* cz;
@@ -704,13 +704,12 @@ static_assert(kPenErrWords == 6, "st[1..6]");
 
 // After the sweep: every octant's tasks done (else err, unless already set);
 // then the next launch's progress base, beyond this one's words, and counters
-// (a context starts with words, base and counters 0: no row done).  One launch
-// for both, where a second one before the sweep took 4 us of each iteration.
+// (a context starts with words, base and counters 0: no row done).  Part of the
+// launch after the switch commit (k_halo).
 struct PencilCounts {
   uint32_t n[8];
 };
-__global__ void k_pencil_done(uint32_t* st, PencilCounts c, uint32_t step) {
-  const uint32_t o = threadIdx.x;
+__device__ __forceinline__ void pencil_done(uint32_t* st, const PencilCounts& c, uint32_t step, uint32_t o) {
   if (o < 8) {
     uint32_t* const q = st + kPenOct * (1 + o);
     const uint32_t done = q[kPenDone];
@@ -1373,19 +1372,53 @@ __global__ void k_commit(T* f, const T* fw, const int32_t* walls, int nwalls,
 // x = 1, both as they were after the previous iteration's sweep (the
 // reference's self send/receive posts last iteration's packed buffers,
 // src/solver.F90:144-171, 535-560).  y/z ghost rows stay zero (MPI_PROC_NULL).
+//
+// The first blocks (sb; they start first) take the snapshot the coupled walls read
+// (wall cells, x in 1..Nx: the exchange writes none of them), and the first one's
+// last wave closes the row sweep (st; null: no row sweep).  As launches of their
+// own these two cost an iteration of a 45 x 38 x 41 pack 8 us of 415, of 16 x 13 x 14
+// boxes 2 of 111; larger images nothing.
 template <typename T>
-__global__ void k_halo(T* f, T* buf_e, T* buf_w, Dims d) {
+struct HaloArgs {
+  T* f;
+  T* buf_e;
+  T* buf_w;
+  T* snap;
+  const int32_t* snap_cell;
+  int nsnap;
+  unsigned sb;              // blocks in front of the exchange's
+  uint32_t* st;
+  PencilCounts counts;
+  uint32_t step;
+};
+
+template <typename T>
+__global__ void k_halo(HaloArgs<T> a, Dims d) {
   const int64_t n = (int64_t)d.Ny * d.Nz * 8 * d.Nc8;
-  f += blockIdx.y * d.rs_f;
-  buf_e += blockIdx.y * d.rs_buf;
-  buf_w += blockIdx.y * d.rs_buf;
+  T* const f = a.f + blockIdx.y * d.rs_f;
+  T* const buf_e = a.buf_e + blockIdx.y * d.rs_buf;
+  T* const buf_w = a.buf_w + blockIdx.y * d.rs_buf;
+  if (blockIdx.x < a.sb) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && a.st && threadIdx.x >= blockDim.x - kWave)
+      pencil_done(a.st, a.counts, a.step, threadIdx.x - (blockDim.x - kWave));
+    const int64_t tot = (int64_t)a.nsnap * 8 * d.Nc8;
+    T* const snap = a.snap + blockIdx.y * d.rs_snap;
+    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < tot; t += (int64_t)a.sb * blockDim.x) {
+      const int l = (int)(t % d.Nc8);
+      const int o = (int)((t / d.Nc8) % 8);
+      const int s = (int)(t / (8 * d.Nc8));
+      snap[t] = f[fat(d, o, a.snap_cell[s]) + l];
+    }
+    return;
+  }
+  const unsigned hb = gridDim.x - a.sb, block = blockIdx.x - a.sb;  // of the exchange
   if (d.Nc8 <= kWave) {
     // one wave per (row, octant), one velocity per lane: the row's storage
     // positions are wave-uniform and all four reads are in flight together
     const int lane = threadIdx.x & (kWave - 1);
     const int wpb = blockDim.x / kWave;
     const int items = d.Ny * d.Nz * 8;
-    for (int it = blockIdx.x * wpb + wave_in_block(); it < items; it += gridDim.x * wpb) {
+    for (int it = block * wpb + wave_in_block(); it < items; it += hb * wpb) {
       const int o = it & 7, r = it >> 3;
       const int j = 1 + r % d.Ny, k = 1 + r / d.Ny;
       const int64_t row = (int64_t)(j + 1) * d.Nxt + (int64_t)(k + 1) * d.Nxyt;
@@ -1400,8 +1433,8 @@ __global__ void k_halo(T* f, T* buf_e, T* buf_w, Dims d) {
     }
     return;
   }
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n;
-       t += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t t = block * (int64_t)blockDim.x + threadIdx.x; t < n;
+       t += (int64_t)hb * blockDim.x) {
     const int l = (int)(t % d.Nc8);
     int64_t r = t / d.Nc8;
     const int o = (int)(r % 8);
@@ -1633,20 +1666,6 @@ __global__ __launch_bounds__(256) void k_walls_coupled(WallArgs<T> a) {
   const int wpb = blockDim.x / kWave;
   for (int idx = blockIdx.x * wpb + wave_in_block(); idx < a.n; idx += gridDim.x * wpb)
     wall_dispatch<T, true>(a, idx, threadIdx.x & (kWave - 1));
-}
-
-template <typename T>
-__global__ void k_snapshot(const T* f, T* snap, const int32_t* cells, int n, Dims d) {
-  const int64_t tot = (int64_t)n * 8 * d.Nc8;
-  f += blockIdx.y * d.rs_f;
-  snap += blockIdx.y * d.rs_snap;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < tot;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int l = (int)(t % d.Nc8);
-    const int o = (int)((t / d.Nc8) % 8);
-    const int s = (int)(t / (8 * d.Nc8));
-    snap[t] = f[fat(d, o, cells[s]) + l];
-  }
 }
 
 // ------------------------------------------------------------------ inlet/outlet, symmetry
@@ -2346,10 +2365,7 @@ int enqueue_t(Ctx& c, State<T>& st, int nsteps, int ev0, const IterMode& im) {
       pa.dc_e = c.s32.f;
       pa.dc_fold = im.fold;
       pa.dc_first = im.first;
-      PencilCounts pc{};
-      for (int q = 0; q < 8; ++q) pc.n[q] = (uint32_t)(g.pen_tasks[q] * pa.units);
       hipLaunchKernelGGL(pencil_kernel<T>(im.dc), dim3(8u * (unsigned)c.pen_waves), dim3(64), 0, c.stream, pa);
-      hipLaunchKernelGGL(k_pencil_done, dim3(1), dim3(64), 0, c.stream, c.pen_state, pc, (uint32_t)g.Nx + 2u);
     }
     const int ng = c.sweep_tiles || c.pencil ? 0 : std::max(1, c.oct_groups);
     const bool conc = ng > 1 && c.side[0] != nullptr;
@@ -2410,14 +2426,17 @@ int enqueue_t(Ctx& c, State<T>& st, int nsteps, int ev0, const IterMode& im) {
       hipLaunchKernelGGL(k_commit<T>, dim3(grid_for((int64_t)g.commit_walls.size(), wpb), R),
                          dim3(wpb * kWave), 0, c.stream, st.f, (const T*)st.fw, c.commit_walls,
                          (int)g.commit_walls.size(), c.wall_pos, c.wall_corner, c.views, d);
-    hipLaunchKernelGGL(k_halo<T>,
-                       dim3(d.Nc8 <= kWave ? grid_for((int64_t)g.Ny * g.Nz * 8, wpb)
-                                           : grid_for((int64_t)g.Ny * g.Nz * 8 * d.Nc8, 256), R),
-                       dim3(256), 0, c.stream, st.f, st.buf_e, st.buf_w, d);
-    if (!g.snap_cell.empty())
-      hipLaunchKernelGGL(k_snapshot<T>, dim3(grid_for((int64_t)g.snap_cell.size() * 8 * d.Nc8, 256), R),
-                         dim3(256), 0, c.stream, (const T*)st.f, st.snap, c.snap_cell,
-                         (int)g.snap_cell.size(), d);
+    HaloArgs<T> ha{st.f, st.buf_e, st.buf_w, st.snap, c.snap_cell, (int)g.snap_cell.size()};
+    const unsigned hb = (unsigned)(d.Nc8 <= kWave ? grid_for((int64_t)g.Ny * g.Nz * 8, wpb)
+                                                  : grid_for((int64_t)g.Ny * g.Nz * 8 * d.Nc8, 256));
+    ha.sb = g.snap_cell.empty() ? 0u : (unsigned)grid_for((int64_t)g.snap_cell.size() * 8 * d.Nc8, 256);
+    if (c.pencil) {
+      ha.st = c.pen_state;
+      ha.step = (uint32_t)g.Nx + 2u;
+      for (int q = 0; q < 8; ++q) ha.counts.n[q] = (uint32_t)(g.pen_tasks[q] * pencil_chunks(d) * R);
+      ha.sb = std::max(ha.sb, 1u);
+    }
+    hipLaunchKernelGGL(k_halo<T>, dim3(ha.sb + hb, R), dim3(256), 0, c.stream, ha, d);
     for (int nf = 1; nf <= 3; ++nf) {
       const int b = g.uncoupled_off[nf - 1], n = g.uncoupled_off[nf] - b;
       if (n == 0) continue;
