@@ -158,7 +158,7 @@ def refined_measurement(p, img, steps, warmup, block, k64, fp64_ms_per_step):
         "correction_iteration_ms": round(it_ms, 4), "correction_sweep_ms": round(sweep_ms, 4),
         "correction_roofline": {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS,
                                 "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4), "bytes_per_update": 12,
-                                "kernel": "k_sweep1<float, false, 2>"},
+                                "kernel": "k_sweep_pencil<float, 2>"},
         "k_rel_diff_vs_fp64_blocks_from_rest": abs(k - k64) / abs(k64) if k64 else abs(k - k64),
         "steps_compared": warmup + steps,
         "fp32_iterations": int(n32)}
