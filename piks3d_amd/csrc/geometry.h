@@ -220,8 +220,9 @@ constexpr int tile_rec_cell(int ns, int tx, int ty, int s) { return 1 + ns + 2 *
 // velocities per octant, the zero slot as the window's end.
 void make_window_relative(Geometry& g, int nc8, int threads);
 
-// Records of the single-launch sweep, from the window-relative hyperplane
-// records: the tasks in octant-major, hyperplane order, kTaskWords words
+// Per-cell records of a single-launch sweep in hyperplane order (no kernel
+// reads them; the tests check the resolved switched reads through them), from
+// the window-relative hyperplane records: the tasks in octant-major, hyperplane order, kTaskWords words
 // each (off[o] the first task of octant o, off[8] the count).  With
 // strips > 1 an octant's tasks go strip by strip (strips equal bands of y,
 // in the octant's y direction), in hyperplane order within a strip: every

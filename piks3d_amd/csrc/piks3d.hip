@@ -129,12 +129,6 @@ __device__ __forceinline__ double wave_sum(double v) {
   return row_sum(x + y);
 }
 
-__device__ __forceinline__ int64_t uniform64(int64_t v) {
-  int lo = __builtin_amdgcn_readfirstlane((int)(v & 0xffffffff));
-  int hi = __builtin_amdgcn_readfirstlane((int)(v >> 32));
-  return ((int64_t)hi << 32) | (uint32_t)lo;
-}
-
 // Read-only data of a kernel loaded through the scalar cache: the constant
 // address space tells the compiler that no store of the kernel can clobber it.
 template <typename T>
@@ -864,7 +858,6 @@ __global__ __launch_bounds__(64) void k_sweep_pencil(PencilArgs<T> args) {
     uint32_t* const own = a->prog + ((size_t)u * 8 + o) * a->npen + pen.id;
     const int32_t sy = osy((int)o), sz = osz((int)o) * (int32_t)a->Ny;
     const ConstPtr<TaskRec> rr = const_ptr(a->rec + pen.rec);
-    const uint32_t last = n - 1u;
     const bool hasy = pen.n >> 31, hasz = (pen.n >> 30) & 1u;
     // The neighbour rows' progress as last seen (lim: the smaller; past the
     // row's end where there is no neighbour or it is finished).  Lane 0 polls
