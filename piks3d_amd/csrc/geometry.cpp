@@ -665,6 +665,7 @@ bool build_tile_schedule(Geometry& g, int TX, int TY, int TZ, int threads) {
   g.tl_ntile = 0;
   g.tl_ndiag = 0;
   g.tl_maxwin = 0;
+  if (g.raster) return false;
   if (TX < 2 || TY < 2 || TZ < 2 || tile_rec_cell(NS, TX, TY, NS) > W || tile_rec_zhalo(NS, 2) > W ||
       NS > 32)
     return false;

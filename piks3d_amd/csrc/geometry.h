@@ -252,8 +252,9 @@ int64_t flow_switched_word(const Geometry& g, int o, int64_t n, int axis);
 // the sweep.  Needs the storage order.
 std::vector<uint32_t> build_nonswept(const Geometry& g, int threads);
 
-// Fill the tiled sweep schedule (tl_*); needs the storage order.  Returns
-// false when a tile shape does not fit the record (the schedule stays empty).
+// Fill the tiled sweep schedule (tl_*); needs the hyperplane storage order.
+// Returns false over raster storage or when a tile shape does not fit the
+// record (the schedule stays empty).
 bool build_tile_schedule(Geometry& g, int tx, int ty, int tz, int threads);
 
 template <typename F>

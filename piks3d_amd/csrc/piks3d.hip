@@ -2285,6 +2285,7 @@ int enqueue_t(Ctx& c, State<T>& st, int nsteps, int ev0, const IterMode& im) {
   }
   TileArgs<T> ta{};
   void (*ktile)(TileArgs<T>) = nullptr;
+  if (c.sweep_tiles && c.pencil) return fail(PIKS_E_STATE, "two sweeps are on");
   if (c.sweep_tiles) {
     ta.f = st.f;
     ta.mom = im.mom;
@@ -2634,11 +2635,17 @@ namespace piks {
 
 namespace {
 
-// Whether the context sweeps in one launch by rows (pencils): the default,
-// unless a setting that shapes the hyperplane or tiled sweep asks for those.
-// PIKS_SWEEP_FLOW=0 turns it off; =1 asks for it and is refused (ctx_create_device)
-// on anything but a single FP64 solve with 64 velocities per octant on a
-// context with its own stream.
+// The context's sweep, decided here for all that is laid out after it.
+//   * Tiles where the parameters (a tuning table's choice), or without a choice
+//     of theirs PIKS_SWEEP_TILES, ask for them and the tiled kernel serves the
+//     context: FP64, at most 64 velocities per octant (the generic kernel is a
+//     forced alternative).
+//   * Else one launch by rows (pencils): the default, unless a setting that
+//     shapes the hyperplane or tiled sweep asks for those.  PIKS_SWEEP_FLOW=0
+//     turns it off; =1 asks for it and is refused (ctx_create_device) on
+//     anything but a single FP64 solve with 64 velocities per octant on a
+//     context with its own stream.
+//   * Else one launch per hyperplane.
 int sweep_choice(Ctx& c) {
   const char* const shaping[] = {"PIKS_XCD_REMAP", "PIKS_SWEEP_BLOCK", "PIKS_SWEEP_TILES", "PIKS_SWEEP_GENERIC",
                                  "PIKS_OCT_GROUPS", "PIKS_OCT_SERIAL", "PIKS_SWEEP_NT", "PIKS_SWEEP_RECIP"};
@@ -2655,6 +2662,11 @@ int sweep_choice(Ctx& c) {
     c.flow_strips = std::atoi(b);
     if (c.flow_strips < 1 || c.flow_strips > 64) return fail(PIKS_E_ARG, "PIKS_FLOW_STRIPS must be 1..64");
   }
+  if (const char* b = std::getenv("PIKS_SWEEP_GENERIC")) c.sweep_generic = std::atoi(b) != 0;
+  if (const char* b = std::getenv("PIKS_SWEEP_TILES")) c.sweep_tiles = std::atoi(b) != 0;
+  if (c.prm.sweep != 0) c.sweep_tiles = c.prm.sweep == 2;
+  if ((int)c.cx.size() > kWave || c.sweep_generic || c.prm.precision == PIKS_PREC_FP32_REFINED) c.sweep_tiles = false;
+  if (c.sweep_tiles) c.flow_req = 0;
   c.pencil = c.flow_req != 0;
   return 0;
 }
@@ -2743,7 +2755,6 @@ int ctx_create_host(const piks_params* p, const uint8_t* raw, int64_t nbytes, Ct
     c->sweep_block = v;
   }
 
-  if (const char* b = std::getenv("PIKS_SWEEP_TILES")) c->sweep_tiles = std::atoi(b) != 0;
   if (const char* b = std::getenv("PIKS_TILE")) {
     int tx = 0, ty = 0, tz = 0;
     if (std::sscanf(b, "%dx%dx%d", &tx, &ty, &tz) != 3 || !tile_kernel<double>(tx, ty) || tz < 2 || tz > 256)
@@ -2752,20 +2763,12 @@ int ctx_create_host(const piks_params* p, const uint8_t* raw, int64_t nbytes, Ct
   }
   if (const char* b = std::getenv("PIKS_GRAPH")) c->use_graph = std::atoi(b) != 0;
   if (const char* b = std::getenv("PIKS_PLANES_FUSED")) c->planes_fused = std::atoi(b) != 0;
-  // the sweep schedule of the parameters (a tuning table's choice) takes
-  // precedence over the environment
-  if (p->sweep == 1) {
-    c->sweep_tiles = false;
-  } else if (p->sweep == 2) {
-    c->sweep_tiles = true;
-    if (p->tile != 0) {
-      const int tx = p->tile & 255, ty = (p->tile >> 8) & 255, tz = (p->tile >> 16) & 0xffff;
-      if (!tile_kernel<double>(tx, ty) || tz < 2 || tz > 256)
-        return fail(PIKS_E_ARG, "tile must be tx | ty << 8 | tz << 16 with tx x ty one of 4x4, 4x2, 8x2, 2x2");
-      c->tile_tx = tx; c->tile_ty = ty; c->tile_tz = tz;
-    }
-  } else if (p->sweep != 0) {
-    return fail(PIKS_E_ARG, "sweep must be 0, 1 or 2");
+  if (p->sweep < 0 || p->sweep > 2) return fail(PIKS_E_ARG, "sweep must be 0, 1 or 2");
+  if (p->sweep == 2 && p->tile != 0) {
+    const int tx = p->tile & 255, ty = (p->tile >> 8) & 255, tz = (p->tile >> 16) & 0xffff;
+    if (!tile_kernel<double>(tx, ty) || tz < 2 || tz > 256)
+      return fail(PIKS_E_ARG, "tile must be tx | ty << 8 | tz << 16 with tx x ty one of 4x4, 4x2, 8x2, 2x2");
+    c->tile_tx = tx; c->tile_ty = ty; c->tile_tz = tz;
   }
   if (const char* b = std::getenv("PIKS_DC_BLOCK")) {
     const int v = std::atoi(b);
@@ -2773,7 +2776,6 @@ int ctx_create_host(const piks_params* p, const uint8_t* raw, int64_t nbytes, Ct
     c->dc_fixed = v;
   }
   if (const char* b = std::getenv("PIKS_SWEEP_RECIP")) c->sweep_recip = std::atoi(b) != 0;
-  if (const char* b = std::getenv("PIKS_SWEEP_GENERIC")) c->sweep_generic = std::atoi(b) != 0;
   if (const char* b = std::getenv("PIKS_OCT_GROUPS")) {
     const int v = std::atoi(b);
     if (v != 1 && v != 2 && v != 4 && v != 8) return fail(PIKS_E_ARG, "PIKS_OCT_GROUPS must be 1, 2, 4 or 8");
@@ -2798,9 +2800,6 @@ int ctx_create_host(const piks_params* p, const uint8_t* raw, int64_t nbytes, Ct
   c->d.rs_fw = (int64_t)c->n_fw;
   c->d.rs_buf = (int64_t)c->n_buf;
   c->d.rs_snap = (int64_t)c->n_snap;
-  // the tiled sweep serves grids of at most 64 velocities per octant and the
-  // generic kernel is a forced alternative
-  if (c->d.Nc8 > kWave || c->sweep_generic || p->precision == PIKS_PREC_FP32_REFINED) c->sweep_tiles = false;
   if (p->precision == PIKS_PREC_FP32_REFINED) {
     c->ns_host = build_nonswept(c->g, host_threads());
     c->n_ns = (int64_t)c->ns_host.size();
