@@ -193,6 +193,12 @@ int set_error(int code, const std::string& msg);
 int ctx_create_host(const piks_params* p, const uint8_t* raw, int64_t nbytes, Ctx** out);
 // Device memory ctx_create_device will allocate (bytes).
 size_t ctx_device_bytes(const Ctx& c);
+// Before the device phase: a context that would take more than `avail` bytes
+// gives up the row sweep for the hyperplane launches where their layout takes
+// less (whole-line slots and one copy of the partial moments per 64 velocities
+// cost memory), unless PIKS_SWEEP_FLOW=1 asks for rows.  Whether it then fits
+// is the caller's to check.
+int ctx_fit(Ctx& c, size_t avail);
 // Device phase: allocate, clear and upload.  stream == nullptr: the context
 // creates its own stream and uses hipMalloc; otherwise it works on `stream`
 // with stream-ordered allocations.  Returns after the uploads have completed

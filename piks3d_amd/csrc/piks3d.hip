@@ -2848,6 +2848,12 @@ size_t ctx_device_bytes(const Ctx& c) {
          R * ((size_t)g.Ny * g.Nz * 8 + 8) + 4 * c.cx.size() * 8 + 64 * 256;
 }
 
+int ctx_fit(Ctx& c, size_t avail) {
+  const bool larger = c.d.vs != c.d.Nc8 || part_units(c) > 1;
+  if (!c.pencil || c.flow_req == 1 || !larger || ctx_device_bytes(c) <= avail) return 0;
+  return use_hyperplanes(c);
+}
+
 // Whether the pencil sweep can run on the context's device: the sweep needs
 // blocks on each of eight XCDs (blocks are dealt to them in turn), numbered
 // as the hardware id reads.  Sizes its launch: the waves per octant (XCD) that
@@ -2944,6 +2950,7 @@ int ctx_create_device(Ctx& c, hipStream_t stream) {
   if (c.own_stream) {
     size_t free_b = 0, total_b = 0;
     HIP_TRY(hipMemGetInfo(&free_b, &total_b));
+    if (int rc = ctx_fit(c, free_b)) return rc;
     const size_t need = ctx_device_bytes(c);
     if (need > free_b)
       return fail(PIKS_E_MEM, "problem needs about " + std::to_string(need >> 20) + " MiB of device memory, " +

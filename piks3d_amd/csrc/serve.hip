@@ -117,7 +117,11 @@ void prep_worker(Server* s) {
       s->prep_q.pop_front();
     }
     Ctx* c = nullptr;
-    const int rc = ctx_create_host(&r->prm, r->image.data(), (int64_t)r->image.size(), &c);
+    int rc = ctx_create_host(&r->prm, r->image.data(), (int64_t)r->image.size(), &c);
+    if (rc == 0 && (rc = ctx_fit(*c, s->budget))) {
+      ctx_destroy(c);
+      c = nullptr;
+    }
     std::lock_guard<std::mutex> lk(s->mu);
     if (rc != 0) {
       r->error_code = rc;

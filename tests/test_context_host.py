@@ -3,7 +3,8 @@ g++ and linked against libpiks3d.so, creates one under each combination of the
 settings that choose the sweep.  Exactly one sweep is on, with the storage
 order and records it reads: tiles where they are asked for and serve the
 context (whatever PIKS_SWEEP_FLOW says), else rows of cells unless a setting
-asks for the hyperplane launches."""
+asks for the hyperplane launches.  A context whose padded slots do not fit the memory there
+is takes the hyperplane launches' layout if that fits."""
 import os
 import shutil
 import subprocess
@@ -74,3 +75,25 @@ def test_generic_kernel_setting_takes_no_tiles(checker):
     # PIKS_SWEEP_GENERIC forces the generic kernel of the hyperplane launches
     got = _host(checker, {"PIKS_SWEEP_GENERIC": "1", "PIKS_SWEEP_TILES": "1"}, 4, 0, 0)
     assert (got["rc"], got["tiles"], got["rows"]) == (0, 0, 0)
+
+
+# FP64 and refined contexts whose slots the rows pad (8, 27) or whose partial
+# moments they keep per 64 velocities (216)
+@pytest.mark.parametrize("nc,precision", [(2, 0), (3, 0), (6, 0), (2, 1), (3, 1)])
+def test_rows_that_do_not_fit_leave_the_hyperplane_layout(checker, nc, precision):
+    rows = _host(checker, {}, nc, precision, 0)
+    hyper = _host(checker, {"PIKS_SWEEP_FLOW": "0"}, nc, precision, 0)
+    assert (rows["rows"], hyper["rows"]) == (1, 0)
+    assert rows["bytes"] > hyper["bytes"]
+    # they fit: nothing changes
+    assert _host(checker, {}, nc, precision, 0, str(rows["bytes"])) == rows
+    # they do not: what PIKS_SWEEP_FLOW=0 lays out, to the last index
+    assert _host(checker, {}, nc, precision, 0, str(rows["bytes"] - 1)) == hyper
+    assert _host(checker, {}, nc, precision, 0, str(hyper["bytes"])) == hyper
+
+
+def test_sweeps_asked_for_stay_whatever_fits(checker):
+    # tiles; and the rows' layout where it is no larger (64 velocities)
+    for env, nc, sweep in (({}, 3, 2), ({"PIKS_SWEEP_FLOW": "1"}, 3, 0), ({}, 4, 0)):
+        got = _host(checker, env, nc, 0, sweep)
+        assert _host(checker, env, nc, 0, sweep, str(got["bytes"] - 1)) == got
