@@ -407,10 +407,11 @@ bool is_stored(const Geometry& g, int i, int j, int k) {
 
 }  // namespace
 
-bool build_pencil_schedule(Geometry& g, int rows, int vs, int threads) {
+bool build_pencil_schedule(Geometry& g, int rows, int vs, int threads, bool wide) {
   const int Nx = g.Nx, Ny = g.Ny, Nz = g.Nz;
   const int64_t npen = (int64_t)Ny * Nz;
   g.raster = true;
+  g.pen_wide = wide = wide || Nx + 1 >= 1 << 14;
   // raster storage order: the stored cells of every row, rows joined in order
   std::vector<int64_t> row0((size_t)npen + 1, 0);
   parallel_for(Nz, threads, [&](int kk) {
@@ -423,7 +424,7 @@ bool build_pencil_schedule(Geometry& g, int rows, int vs, int threads) {
   for (int64_t q = 0; q < npen; ++q) row0[(size_t)q + 1] += row0[(size_t)q];
   const int64_t ns = g.nstore = row0[(size_t)npen];
   if (8 * (ns + 1) >= (int64_t)Geometry::kPenFw || (int64_t)g.ncorner * 8 >= (int64_t)Geometry::kPenFw ||
-      Nx + 1 >= 1 << 14)
+      Nx + 1 >= 1 << 26)  // a row's partial moments and moments: 31-bit byte offsets
     return false;
   std::vector<int32_t>& pos = g.pos[0];
   pos.assign((size_t)g.Ntotal, (int32_t)ns);
@@ -502,7 +503,7 @@ bool build_pencil_schedule(Geometry& g, int rows, int vs, int threads) {
           if (g.lab[(size_t)c] != FLUID) continue;
           const uint32_t cc = g.code[(size_t)c];
           uint32_t w0 = rel(pos[(size_t)c]) | ((cc >> (3 * o)) & 7u) << 28;
-          uint32_t w1 = (uint32_t)i | (uint32_t)(oi + 1) << 14;
+          uint32_t w1 = wide ? (uint32_t)(oi + 1) : (uint32_t)i | (uint32_t)(oi + 1) << 14;
           const bool x1 = oi - 1 >= 1 && g.lab[(size_t)(c - dx)] == FLUID;
           const bool x2 = oi - 2 >= 1 && g.lab[(size_t)(c - 2 * dx)] == FLUID;
           r[6] = x1 ? 0u : rel(pos[(size_t)(c - dx)]) * 8u;

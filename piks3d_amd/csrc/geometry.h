@@ -153,7 +153,9 @@ struct Geometry {
   //       kPenSpecial (a far source, or a wait at distance 2)
   //   [1] x index i | (oriented x + 1) << 14 | kPenX1Reg, kPenX2Reg (the x
   //       upwind value at distance 1, 2 is the row's own result) | kPenWaitY,
-  //       kPenWaitZ (the neighbour at distance 1 is swept: wait for its row)
+  //       kPenWaitZ (the neighbour at distance 1 is swept: wait for its row);
+  //       with rows of 2^14 - 1 cells and more (pen_wide), whose two x do not
+  //       fit, oriented x + 1 alone in bits 0-27
   //   [2..5] the y upwind sources at distance 1 and 2, then z: offsets in
   //       bytes of 8-byte elements, or kPenFar (beyond every window): a storage
   //       row octant * (nstore + 1) + index, or with kPenFw a corner store
@@ -178,6 +180,7 @@ struct Geometry {
   static constexpr uint32_t kPenFar = 1u << 31, kPenFw = 1u << 30, kPenWaitY2 = 1, kPenWaitZ2 = 2;
   std::vector<Pencil> pen;
   std::vector<uint32_t> pen_rec;
+  bool pen_wide = false;
   int64_t pen_off[9] = {};
   int64_t pen_tasks[8] = {};
 
@@ -194,9 +197,10 @@ int build_geometry(const GeomInput& in, const uint8_t* raw, int64_t nbytes, Geom
 void build_sweep_schedule(Geometry& g, int threads);
 
 // Fill the raster storage order and the pencil schedule (pen, pen_rec), with
-// strips of `rows` y rows and vs elements per slot.  False if the image is beyond the records' limits
-// (the hyperplane schedule is then built over it).
-bool build_pencil_schedule(Geometry& g, int rows, int vs, int threads);
+// strips of `rows` y rows and vs elements per slot; with `wide` the records of
+// long rows whatever their length.  False if the image is beyond the records'
+// limits (the hyperplane schedule is then built over it).
+bool build_pencil_schedule(Geometry& g, int rows, int vs, int threads, bool wide = false);
 
 // Dword positions inside the tiled sweep's records (tile of tx * ty cells per
 // plane, ns = tx * ty slots, slot s = b * tx + a for oriented offsets a, b).

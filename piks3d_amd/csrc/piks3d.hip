@@ -760,7 +760,11 @@ struct alignas(8) PenNbr {
   uint32_t nb[4], x[2];
 };
 
-template <typename T, int kDC>
+// kWide: the records of rows too long for two x in a word (Geometry::pen_wide).
+// A variant of its own, since the moments' offset then takes two more scalar
+// operations per task, on scalars held across the row.  16400 x 6 x 6, 64
+// velocities: 66.4 ms per iteration with hyperplane launches, 9.4 by rows.
+template <typename T, int kDC, bool kWide>
 __global__ __launch_bounds__(64) void k_sweep_pencil(PencilArgs<T> args) {
   // Arguments are read where they are used (args_now), not held in registers
   // across the row loop: the row loop's own scalars fill the SGPRs.
@@ -874,7 +878,7 @@ __global__ __launch_bounds__(64) void k_sweep_pencil(PencilArgs<T> args) {
       pz = hasz && vz <= Nx ? vz : kAll;
       lim = min(py, pz);
     };
-    auto ox1 = [](uint32_t w1) -> int32_t { return (int32_t)((w1 >> 14) & 0x3fffu); };
+    auto ox1 = [](uint32_t w1) -> int32_t { return (int32_t)(kWide ? w1 & 0x0fffffffu : (w1 >> 14) & 0x3fffu); };
     auto publish = [&](uint32_t v) {
       // every lane writes the same word
       __hip_atomic_store(own, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -897,7 +901,13 @@ __global__ __launch_bounds__(64) void k_sweep_pencil(PencilArgs<T> args) {
     // byte offset of a source word (in 8-byte elements)
     auto src_off = [](uint32_t w) -> uint32_t { return sizeof(T) == 8 ? w : w >> 1; };
     auto self_off = [](uint32_t w0) -> uint32_t { return (w0 & 0x0fffffffu) << kSelf; };
-    auto mom_off = [](uint32_t w1) -> uint32_t { return (w1 & 0x3fffu) << 5; };
+    auto mom_off = [&](uint32_t w1) -> uint32_t {
+      if constexpr (kWide) {
+        const uint32_t x = w1 & 0x0fffffffu;
+        return (osx((int)o) > 0 ? x : (uint32_t)Nx + 1u - x) << 5;
+      }
+      return (w1 & 0x3fffu) << 5;
+    };
     auto ld_mom = [&](uint32_t w1) -> Mom {
       return *(ConstPtr<Mom>)((ConstPtr<char>)momr + mom_off(w1));
     };
@@ -2214,11 +2224,13 @@ SweepKernel<T> sweep_kernel_dc(const Ctx& c, int rb) {
   }
 }
 
-// The pencil sweep's kernel for a defect-correction role (IterMode::dc).
+// The pencil sweep's kernel for a defect-correction role (IterMode::dc) and
+// the context's records (Geometry::pen_wide).
 template <typename T>
-auto pencil_kernel(int dc) -> void (*)(PencilArgs<T>) {
-  if constexpr (sizeof(T) == sizeof(float)) return k_sweep_pencil<float, 2>;
-  else return dc ? k_sweep_pencil<double, 1> : k_sweep_pencil<double, 0>;
+auto pencil_kernel(int dc, bool wide) -> void (*)(PencilArgs<T>) {
+  if constexpr (sizeof(T) == sizeof(float)) return wide ? k_sweep_pencil<float, 2, true> : k_sweep_pencil<float, 2, false>;
+  else if (dc) return wide ? k_sweep_pencil<double, 1, true> : k_sweep_pencil<double, 1, false>;
+  else return wide ? k_sweep_pencil<double, 0, true> : k_sweep_pencil<double, 0, false>;
 }
 
 // Units of 64 velocities per octant.
@@ -2359,7 +2371,7 @@ int enqueue_t(Ctx& c, State<T>& st, int nsteps, int ev0, const IterMode& im) {
       pa.dc_e = c.s32.f;
       pa.dc_fold = im.fold;
       pa.dc_first = im.first;
-      hipLaunchKernelGGL(pencil_kernel<T>(im.dc), dim3(8u * (unsigned)c.pen_waves), dim3(64), 0, c.stream, pa);
+      hipLaunchKernelGGL(pencil_kernel<T>(im.dc, g.pen_wide), dim3(8u * (unsigned)c.pen_waves), dim3(64), 0, c.stream, pa);
     }
     const int ng = c.sweep_tiles || c.pencil ? 0 : std::max(1, c.oct_groups);
     const bool conc = ng > 1 && c.side[0] != nullptr;
@@ -2863,9 +2875,9 @@ int pencil_probe(Ctx& c, bool* usable) {
   int per_cu = 0, dev = 0;
   const bool refined = c.prm.precision == PIKS_PREC_FP32_REFINED;
   if (refined)
-    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (k_sweep_pencil<float, 2>), 64, 0));
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (k_sweep_pencil<float, 2, false>), 64, 0));
   else
-    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (k_sweep_pencil<double, 0>), 64, 0));
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (k_sweep_pencil<double, 0, false>), 64, 0));
   hipDeviceProp_t prop;
   HIP_TRY(hipGetDevice(&dev));
   HIP_TRY(hipGetDeviceProperties(&prop, dev));
