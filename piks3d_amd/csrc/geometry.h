@@ -90,7 +90,8 @@ struct Geometry {
   // family's signs, then k, then j, so that one hyperplane of a sweep is one
   // contiguous range.  pos[F] maps a cell to its index in family F's order.
   // With the pencil schedule (raster) every octant keeps its cells in one
-  // raster order instead (k, then j, then i), held in pos[0].
+  // raster order instead (k, then j, then i; or j, then k, then i where only
+  // that keeps the rows' windows within 32-bit offsets), held in pos[0].
   int64_t nstore = 0;
   bool raster = false;
   std::vector<int32_t> pos[4];
