@@ -124,6 +124,7 @@ def refined_measurement(p, img, steps, warmup, block, k64, fp64_ms_per_step):
     os.environ["PIKS_DC_BLOCK"] = "1"
     with Solver(p, img, precision="fp32") as s:
         nf, nc = s.info.nfluid, s.info.nc8 * 8
+        rows = s.sweep_kind() == "rows"
         s.iterate(warmup)
         s.chk_converge()
         os.environ.pop("PIKS_DC_BLOCK")
@@ -158,7 +159,7 @@ def refined_measurement(p, img, steps, warmup, block, k64, fp64_ms_per_step):
         "correction_iteration_ms": round(it_ms, 4), "correction_sweep_ms": round(sweep_ms, 4),
         "correction_roofline": {"bound": "hbm", "achieved": round(ach, 1), "peak": HBM_PEAK_GBS,
                                 "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4), "bytes_per_update": 12,
-                                "kernel": "k_sweep_pencil<float, 2>"},
+                                "kernel": "k_sweep_pencil<float, 2, false>" if rows else "k_sweep1<float, false, 2>"},
         "k_rel_diff_vs_fp64_blocks_from_rest": abs(k - k64) / abs(k64) if k64 else abs(k - k64),
         "steps_compared": warmup + steps,
         "fp32_iterations": int(n32)}
@@ -606,7 +607,7 @@ def main():
     log("set-up %.1f s: Nfluid %d, walls %d, corners %d, device memory %.1f GB" % (
         time.perf_counter() - t, info.nfluid, info.nwall, info.ncorner, info.device_bytes / 1e9))
     nc = info.nc8 * 8
-    flow = info.sweep_path == 2
+    flow = s.sweep_kind() == "rows"
     log("sweep: %s" % ("one launch per iteration (k_sweep_pencil)" if flow else "one launch per hyperplane"))
     if args.warmup:
         s.iterate(args.warmup)

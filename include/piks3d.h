@@ -166,6 +166,12 @@ int piks_get_labels(void* ctx, int32_t* labels);
 
 int piks_get_info(void* ctx, piks_info* info);
 
+/* The sweep a context of any precision, velocity grid and number of Kn runs:
+ * *kind = 0 one launch per hyperplane, 1 tiles, 2 rows of cells, the whole
+ * sweep in one launch (piks_info.sweep_path says 2 for one kind of context
+ * only).  No counterpart in the reference. */
+int piks_get_sweep(void* ctx, int32_t* kind);
+
 /* Host-only image preprocessing (no device needed): the labelled image of
  * src/physicalGrid.F90:251-671 (Ntotal int32 into labels, may be NULL) and
  * its counts in info (nx..ntotal, nc8 = 0, nwall, ncorner, nfluid,

@@ -99,6 +99,7 @@ _API = {
     "piks_get_info": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(PiksInfo)]),
     "piks_preprocess": (ctypes.c_int, [ctypes.POINTER(PiksParams), ctypes.c_void_p, ctypes.c_int64,
                                        ctypes.c_void_p, ctypes.POINTER(PiksInfo)]),
+    "piks_get_sweep": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int32)]),
     "piks_last_timing": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_double)]),
     "piks_destroy": (ctypes.c_int, [ctypes.c_void_p]),
     "piks_last_error": (ctypes.c_char_p, []),
@@ -214,6 +215,13 @@ class Solver:
         info = PiksInfo()
         _check(lib().piks_get_info(self._h, ctypes.byref(info)))
         return info
+
+    def sweep_kind(self):
+        """The sweep this context runs, whatever its precision, velocity grid
+        and number of Kn: "hyperplanes", "tiles" or "rows"."""
+        kind = ctypes.c_int32()
+        _check(lib().piks_get_sweep(self._h, ctypes.byref(kind)))
+        return ("hyperplanes", "tiles", "rows")[kind.value]
 
     def iterate(self, n=1):
         _check(lib().piks_iterate(self._h, int(n)))

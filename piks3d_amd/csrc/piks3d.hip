@@ -3505,6 +3505,13 @@ int piks_get_info(void* ctx, piks_info* info) {
   return 0;
 }
 
+int piks_get_sweep(void* ctx, int32_t* kind) {
+  if (!ctx || !kind) return fail(PIKS_E_ARG, "null argument");
+  const Ctx& c = *static_cast<Ctx*>(ctx);
+  *kind = c.pencil ? 2 : c.sweep_tiles ? 1 : 0;
+  return 0;
+}
+
 int piks_preprocess(const piks_params* p, const uint8_t* raw_image, int64_t image_bytes,
                     int32_t* labels, piks_info* info) {
   g_err.clear();
