@@ -122,6 +122,8 @@ struct Ctx {
   bool pencil = false;                // in use
   int pen_rows = 0;                   // y rows per strip
   int pen_waves = 0;                  // waves launched per octant
+  uint32_t pen_spin = 1u << 20;       // polls before a wait gives up: seconds, far beyond any
+                                      // wait of a sweep
   TaskRec* pen_rec = nullptr;         // Geometry::pen_rec
   Geometry::Pencil* pen_list = nullptr;  // Geometry::pen
   uint32_t* pen_prog = nullptr;       // [unit][octant][row]: progress

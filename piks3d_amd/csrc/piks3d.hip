@@ -2366,7 +2366,7 @@ int enqueue_t(Ctx& c, State<T>& st, int nsteps, int ev0, const IterMode& im) {
       pa.rec = c.pen_rec;
       pa.pens = c.pen_list;
       pa.mom = im.mom;
-      pa.spin = 1u << 20;  // seconds of polls, far beyond any wait of a sweep
+      pa.spin = c.pen_spin;
       pa.dc_r = c.r32.f;
       pa.dc_e = c.s32.f;
       pa.dc_fold = im.fold;
@@ -2918,17 +2918,21 @@ int pencil_failure(const uint32_t* err) {
                 " tasks"
           : "a dependency wait gave up (octant " + std::to_string(err[1]) + ", task " + std::to_string(err[2]) +
                 " of row " + std::to_string(err[3]) + ", unit " + std::to_string(err[4]) + ")";
-  return fail(PIKS_E_HIP, "single-launch sweep: " + what + "; the state is not valid any more");
+  return fail(PIKS_E_HIP, "single-launch sweep: " + what + "; the iteration's result is not valid");
 }
 
 // A failed wait of the pencil sweep, after the context's stream has been
-// synchronised: the iteration's result, and so the context's state, is not
-// valid.
+// synchronised: the iteration's result is not valid.  It is reported once: the
+// flag would end the next iterations' waits too, and their launches find the
+// counters and words they need whatever this one left (pencil_done).
 int pencil_check(Ctx& c) {
   if (!c.pencil) return 0;
-  uint32_t err[6] = {0, 0, 0, 0, 0, 0};
+  uint32_t err[kPenErrWords] = {};
   HIP_TRY(hipMemcpy(err, c.pen_state + 1, sizeof(err), hipMemcpyDeviceToHost));
-  return err[0] ? pencil_failure(err) : 0;
+  if (!err[0]) return 0;
+  const uint32_t none[kPenErrWords] = {};
+  HIP_TRY(hipMemcpy(c.pen_state + 1, none, sizeof(none), hipMemcpyHostToDevice));
+  return pencil_failure(err);
 }
 
 // Average sweep tasks (swept cell, octant) per oriented hyperplane.
