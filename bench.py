@@ -264,7 +264,7 @@ def kn_sweep_bench(args):
     """Multi-RHS Knudsen sweep: one 160^3 Gaussian-random-field image
     (correlation length 5 voxels, porosity 0.25, percolating in x), 32 Kn
     log-spaced over [1e-3, 10], 8^3 velocities, solved as groups of right-hand
-    sides sharing the geometry (one sweep launch per hyperplane for a group),
+    sides sharing the geometry (one sweep launch per iteration for a group),
     in --precision (fp32: the FP64 defect correction with FP32 correction
     iterations); a few Kn are re-solved in plain FP64 for the same number of
     iterations and compared."""

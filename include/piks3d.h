@@ -181,9 +181,8 @@ int piks_preprocess(const piks_params* p, const uint8_t* raw_image, int64_t imag
 
 /* Several right-hand sides on one geometry: nrhs solves of the same image,
  * velocity grid and parameters that differ only in Kn (kn[0..nrhs-1]; p->kn is
- * ignored), advanced together by piks_iterate with one sweep launch per
- * hyperplane for all of them (each task's geometry record is read once for
- * all right-hand sides).  No counterpart in the reference, which solves one Kn
+ * ignored), advanced together by piks_iterate with one sweep launch for all
+ * of them.  No counterpart in the reference, which solves one Kn
  * per run; each right-hand side's iterates are those of piks_create with its
  * Kn.  piks_chk_converge_multi fills out[3*r + 0..2] = mass, permeability,
  * error of right-hand side r (src/output.F90:151-155 for each); the other

@@ -385,7 +385,7 @@ class Server:
 
 class MultiSolver(Solver):
     """Several Knudsen numbers on one geometry (piks_create_multi): one
-    context, one sweep per hyperplane for all right-hand sides."""
+    context, one sweep launch for all right-hand sides."""
 
     def __init__(self, params: Params, image, kn_values, precision=None, exact_order=None, device=None):
         self.params = params

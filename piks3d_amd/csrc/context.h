@@ -118,7 +118,7 @@ struct Ctx {
   // pencil sweep (k_sweep_pencil): the whole sweep in one launch, octant o on
   // XCD o, rows of cells along x claimed in dependency order
   int flow_req = -1;                  // -1 where it applies, 0 off, 1 required
-  int flow_strips = 0;                // strips of y rows asked for (0: by size)
+  int flow_strips = 0;                // strips of y rows asked for (0: one)
   bool pencil = false;                // in use
   int pen_rows = 0;                   // y rows per strip
   int pen_waves = 0;                  // waves launched per octant

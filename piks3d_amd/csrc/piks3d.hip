@@ -645,17 +645,20 @@ __global__ __launch_bounds__(64) void k_sweep1_rhs(SweepArgs<T> a) { sweep1_task
 //
 // What bounds it: at 200^3 the bytes between L2 and memory (rows are read again
 // for the next two diagonals; 11.5 ms where one read and one write of the
-// octants' slots take about 8.3 ms at a large copy's rate), at small images the
-// chain of rows, (Ny + Nz) hops of a few tasks each.  Sweep of one iteration,
-// one launch per hyperplane or per-cell flags before / rows: 32^3 pack, 27
-// velocities 0.54 / 0.20 ms, 45 x 38 x 41 0.46 / 0.30, sphere in 64^3 1.21 /
-// 0.84, 108 x 97 x 101 2.51 / 1.85, 96^3 with 216 velocities 16.1 / 6.0, 200^3
-// 16.5 / 11.5, six Kn in 112^3 16.3 / 10.3, 128^3 refined 8.7 / 2.9.  With the
-// octants' counters and words in shared lines: 32^3 0.24, 45 x 38 x 41 0.34,
-// 64^3 0.87.
+// swept slots, 30.4 GB, take 6.3 ms at a large copy's 4.85 TB/s), at small
+// images the chain of rows, (Ny + Nz) hops of a few tasks each; everywhere a
+// task's 79 scalar instructions beside 74 vector ones (54 to 76 scalar
+// registers are spilled to vector lanes).  Sweep of one iteration, one launch
+// per hyperplane or per-cell flags before / rows: 32^3 pack, 27 velocities
+// 0.54 / 0.19 ms, 45 x 38 x 41 0.46 / 0.29, sphere in 64^3 1.21 / 0.82, 108 x
+// 97 x 101 2.51 / 1.86, 96^3 with 216 velocities 16.1 / 6.0, 200^3 16.5 / 11.5,
+// six Kn in 112^3 16.3 / 10.2, 128^3 refined 8.7 / 2.8.  With the octants'
+// counters and words in shared lines: 32^3 0.24, 45 x 38 x 41 0.34, 64^3 0.87.
 //
 // A re-poll of a row's progress waits 20 x 64 cycles: fewer polls in flight
-// leave the memory system to the rows being waited for.
+// leave the memory system to the rows being waited for.  It matters little:
+// 4, 10, 20, 40 took 0.191, 0.191, 0.191, 0.199 ms on the 32^3 pack, 0.294,
+// 0.293, 0.289, 0.293 on 45 x 38 x 41, the same within 1 % on larger images.
 constexpr int kPenSleep = 20;
 
 template <typename T>
@@ -2244,9 +2247,13 @@ inline size_t pencil_words(const Geometry& g) { return ((size_t)g.Ny * g.Nz + 31
 // pencil sweep; the other sweeps add their velocity passes in place).
 inline int part_units(const Ctx& c) { return c.pencil ? (int)pencil_chunks(c.d) : 1; }
 
-// Units whose rows are taken together: one unit's rows keep about as many
-// waves busy as a strip's diagonal holds rows times the rows a wave-long
-// diagonal chain overlaps, so small images interleave several units.
+// Units whose rows are taken together, row by row: as many as fill the waves if
+// one unit's rows keep 16 waves busy for every row of its longest diagonal (so
+// one unit from about 24 rows on).  That estimate is too high: all units
+// together were faster wherever there are several, sweep ms with this rule /
+// all together: 96^3 with 216 velocities (4 units) 5.98 / 5.03, 48^3 1.39 /
+// 0.82, four Kn in 40^3 with 27 velocities 0.93 / 0.51, six Kn in 112^3 10.2 /
+// 10.0; one unit at a time is as this rule from 40^3 on.
 inline uint32_t pencil_group(const Ctx& c, uint32_t units) {
   const int64_t rows = std::min<int64_t>(c.pen_rows, std::min(c.g.Ny, c.g.Nz));
   const int64_t busy = std::max<int64_t>(1, rows * 16);
@@ -2886,8 +2893,15 @@ int pencil_probe(Ctx& c, bool* usable) {
     for (int o = 0; o < 8; ++o) rows = std::max<int64_t>(rows, c.g.pen_off[o + 1] - c.g.pen_off[o]);
     // Twelve waves per CU: fewer leave memory latency uncovered, more spread the
     // rows in flight beyond what the L2 holds and make each trail its neighbours
-    // longer.  200^3 pack sweep at 8, 10, 12, 20 waves per CU: 12.6, 11.7, 11.5,
-    // 13.3 ms; 64^3: 0.88, 0.86, 0.87, 1.00 ms (shared counter lines still).
+    // longer.  Sweep at 4, 8, 10, 12, 16, 20 waves per CU, ms:
+    //   200^3                   19.2   12.6   11.6   11.5   12.1   13.2
+    //   108 x 97 x 101          2.82   1.99   1.88   1.86   1.98   2.13
+    //   64^3 sphere             1.08   0.84   0.82   0.82   0.86   0.90
+    //   96^3, 216 velocities    9.26   6.46   6.07   5.98   6.30   6.77
+    //   112^3, six Kn           15.5   10.9   10.3   10.2   10.7   11.4
+    //   128^3, refined          5.17   3.34   3.03   2.85   2.78   2.79
+    //   45 x 38 x 41            0.314  0.289  0.293  0.292  0.289  0.293
+    //   32^3, 27 velocities     0.204  0.194  0.193  0.192  0.192  0.194
     const int64_t fit = std::max<int64_t>(8, (int64_t)std::min(per_cu, 12) * prop.multiProcessorCount / 8);
     c.pen_waves = (int)std::max<int64_t>(8, std::min<int64_t>(fit, rows * c.nrhs * pencil_chunks(c.d)));
   }
